@@ -125,11 +125,32 @@ def test_runs_match_oracle(size, target):
         assert bad == 0, f"{text} at {size}, target {target}: {bad} bytes differ"
 
 
+@pytest.mark.parametrize("target", [(7, 0), (7, 9)], ids=["rgba8", "rgba_half"])
+@pytest.mark.parametrize("size", [(603, 401), (16, 2000), (2000, 16), (80, 64)], ids=lambda s: f"{s[0]}x{s[1]}")
+@pytest.mark.parametrize("text", ["c p2047 l2047", "c t9 p2049 l2048 p700 l600 p1", "c p70000", "c l5000 p5000 l64"])
+def test_long_runs_match_oracle(text, size, target):
+    """Runs around the length from which tiles walk only the groups marked
+    for them, and ones of many groups; long, steep, flat and thick lines and
+    discs across tile edges."""
+    for seed in (100, 101, 102):
+        print(f"{size} {target} {text} {seed}", flush=True)
+        program = _parse(text)
+        with OracleExecutor():
+            ctx, want = _record(program, seed, size, target)
+            _finish(ctx)
+        pf.lib().pfxSetExecutor(None, None)
+        ctx, got = _record(program, seed, size, target)
+        _finish(ctx)
+        bad = np.count_nonzero(want != got)
+        assert bad == 0, f"{text} at {size}, target {target}, seed {seed}: {bad} bytes differ"
+
+
 def test_runs_of_several_frames_replayed():
     """Frames whose k-th runs differ in kind, in one job: the first run and
     two replays of its graph equal the oracle's frames."""
     L = pf.lib()
-    frames = [(PROGRAMS[6], (64, 48)), (PROGRAMS[5], (130, 17)), (PROGRAMS[7], (33, 33)), ("c t6", (40, 40)), ("c l9 i2", (50, 20))]
+    frames = [(PROGRAMS[6], (64, 48)), (PROGRAMS[5], (130, 17)), (PROGRAMS[7], (33, 33)), ("c t6", (40, 40)), ("c l9 i2", (50, 20)),
+              ("c p3000 l3000", (300, 200)), ("c r4 p2500", (400, 300))]
     want = []
     with OracleExecutor():
         for k, (text, size) in enumerate(frames):
