@@ -117,6 +117,8 @@ int pfdExecuteFrameNoAlloc(const PFFframe* frame);
  * ignored). */
 void* pfdHostAlloc(size_t bytes);
 void  pfdHostFree(void* p);
+/* memcpy between host buffers, split over a few threads from 256 KiB on. */
+void  pfdHostCopy(void* dst, const void* src, size_t bytes);
 
 /* Device copies of host bytes that outlive frames (no reference
  * counterpart): render lists keep their recorded vertices resident, and

@@ -1808,8 +1808,12 @@ constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
 // One block scans an array in place (exclusive) and writes its total;
 // with a second array (b != nullptr) it scans that one too.
+// hostOut (page-locked host memory, or null) takes the totals and the
+// clip-list count too, so that a sizing run reads them without copies.
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(uint32_t* __restrict__ a, uint32_t* __restrict__ b, uint32_t nb,
-                                                           uint32_t* __restrict__ totalOut) {
+                                                           uint32_t* __restrict__ totalOut,
+                                                           const uint32_t* __restrict__ clipCount,
+                                                           uint32_t* __restrict__ hostOut) {
     __shared__ uint32_t lds[64];
     for (int which = 0; which < 2; which++) {
         uint32_t* arr = which ? b : a;
@@ -1826,8 +1830,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(uint32_t* __restrict_
             for (int i = 0; i < SCAN_ITEMS; i++) { if (base + i < nb) arr[base + i] = ex; ex += v[i]; }
             carry += total;
         }
-        if (threadIdx.x == 0) totalOut[which] = carry;
+        if (threadIdx.x == 0) {
+            totalOut[which] = carry;
+            if (hostOut) hostOut[which] = carry;
+        }
     }
+    if (threadIdx.x == 0 && hostOut) hostOut[2] = *clipCount;
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t n, uint32_t v) {
@@ -2632,14 +2640,20 @@ __device__ __forceinline__ void raster_tiles(const RasterArgs& A) {
     const uint32_t wg = xcd_chunked(blockIdx.x, gridDim.x);
     const uint32_t tile = (NB == 1) ? wg * 4 + wave : wg;
     if (tile >= A.numTiles) return;
+    // Four slots per tile, one per wave; a tile of one wave fills them all.
     uint32_t* fragOut = A.tileFrags + (size_t)tile * 4 + (NB == 1 ? 0 : wave);
     const bool lead = (threadIdx.x & 63) == 0;
+    const auto count = [&](uint32_t frags) {
+        if (!lead) return;
+        if (NB == 1) *reinterpret_cast<uint4*>(fragOut) = make_uint4(frags, 0u, 0u, 0u);
+        else *fragOut = frags;
+    };
     const uint32_t frame = A.tileFrame[tile];
     const DTileFrame sg = A.tileDesc[frame];
-    if (!sg.active) { if (lead) *fragOut = 0u; return; }
+    if (!sg.active) { count(0u); return; }
     const DFrame& F = sg.F;
     const uint32_t e0 = A.tileBegin[tile], e1 = A.tileEnd[tile];
-    if (e0 == e1 && !sg.clear) { if (lead) *fragOut = 0u; return; }
+    if (e0 == e1 && !sg.clear) { count(0u); return; }
     const uint32_t local = tile - F.tileBase;
     const int tx = (int)(local % F.tilesX), ty = (int)(local / F.tilesX);
     uint32_t frags = 0;
@@ -2652,7 +2666,7 @@ __device__ __forceinline__ void raster_tiles(const RasterArgs& A) {
         constexpr bool QUAD = TS == 16 && K == 1 && MODE == 0;
         frags += raster_block<MODE, PHONG, K, TK, QUAD, WIN, HIZ>(A, F, sg, frame, bx0, by0, e0, e1, Q, b);
     }
-    if (lead) *fragOut = frags;
+    count(frags);
 }
 
 template <int TS, int MODE, bool PHONG, int K, int TK, bool HIZ>
@@ -3943,7 +3957,7 @@ __device__ bool project_line(const PFFstate& st, const PFFline& l, float* h1, fl
 __global__ __launch_bounds__(256) void k_line_setup(const PFFline* __restrict__ lines, uint32_t n,
                                                     const PFFstate* __restrict__ states, DLineScr* __restrict__ out) {
     const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= n || !lines[g].groupStart) return;
+    if (g >= n || (g > 0 && !lines[g].groupStart)) return;     // the first line of a job starts a group
     bool dead = false;
     for (uint32_t i = g; i < n && (i == g || !lines[i].groupStart); i++) {
         const PFFline l = lines[i];
@@ -4314,6 +4328,35 @@ constexpr uint32_t COPY_CHUNK = 16384;
 
 constexpr uint32_t COPY_BLOCKS = 128;
 
+// Chunk c (of the launch) of region r: 16 bytes per lane and load where both
+// ends allow it.
+__device__ __forceinline__ void copy_chunk(const CopyRegion& r, uint32_t c) {
+    const size_t at = (size_t)(c - r.firstChunk) * COPY_CHUNK;
+    if (at >= r.bytes) return;
+    const uint32_t len = (uint32_t)(r.bytes - at < COPY_CHUNK ? r.bytes - at : COPY_CHUNK);
+    const uint8_t* src = r.src + at;
+    uint8_t* dst = r.dst + at;
+    const uintptr_t ends = (uintptr_t)dst | (uintptr_t)src;
+    uint32_t done = 0;
+    if ((ends & 15u) == 0) {
+        const uint32_t q = len / 16;
+        Words4 v[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (threadIdx.x + 256 * k < q) v[k] = reinterpret_cast<const Words4*>(src)[threadIdx.x + 256 * k];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (threadIdx.x + 256 * k < q) reinterpret_cast<Words4*>(dst)[threadIdx.x + 256 * k] = v[k];
+        done = q * 16;
+    } else if ((ends & 3u) == 0) {
+        const uint32_t q = len / 4;
+        for (uint32_t i = threadIdx.x; i < q; i += 256)
+            reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[i];
+        done = q * 4;
+    }
+    for (uint32_t i = done + threadIdx.x; i < len; i += 256) dst[i] = src[i];
+}
+
 __global__ __launch_bounds__(256) void k_copy_out(const CopyRegion* __restrict__ regions, uint32_t n, uint32_t chunks) {
     uint32_t lo = 0;
     for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
@@ -4322,31 +4365,39 @@ __global__ __launch_bounds__(256) void k_copy_out(const CopyRegion* __restrict__
             const uint32_t mid = (lo + hi) >> 1;
             if (regions[mid].firstChunk <= c) lo = mid; else hi = mid;
         }
-        const CopyRegion r = regions[lo];
-        const size_t at = (size_t)(c - r.firstChunk) * COPY_CHUNK;
-        if (at >= r.bytes) continue;
-        const uint32_t len = (uint32_t)(r.bytes - at < COPY_CHUNK ? r.bytes - at : COPY_CHUNK);
-        const uint8_t* src = r.src + at;
-        uint8_t* dst = r.dst + at;
-        uint32_t done = 0;
-        if (((uintptr_t)dst & 15u) == 0) {
-            const uint32_t q = len / 16;
-            Words4 v[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++)
-                if (threadIdx.x + 256 * k < q) v[k] = reinterpret_cast<const Words4*>(src)[threadIdx.x + 256 * k];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++)
-                if (threadIdx.x + 256 * k < q) reinterpret_cast<Words4*>(dst)[threadIdx.x + 256 * k] = v[k];
-            done = q * 16;
-        } else if (((uintptr_t)dst & 3u) == 0) {
-            const uint32_t q = len / 4;
-            for (uint32_t i = threadIdx.x; i < q; i += 256)
-                reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[i];
-            done = q * 4;
-        }
-        for (uint32_t i = done + threadIdx.x; i < len; i += 256) dst[i] = src[i];
+        copy_chunk(regions[lo], c);
     }
+}
+
+// The same for a few regions, handed over with the launch: the uploads of a
+// frame's inputs and tables, read from page-locked host memory by the kernel
+// (a copy command and a round trip each before).
+constexpr uint32_t COPY_INLINE = 24;
+struct CopyList {
+    uint32_t   n, chunks;
+    CopyRegion r[COPY_INLINE];
+};
+__global__ __launch_bounds__(256) void k_copy_list(CopyList L) {
+    uint32_t at = 0;
+    for (uint32_t c = blockIdx.x; c < L.chunks; c += gridDim.x) {
+        while (at + 1 < L.n && L.r[at + 1].firstChunk <= c) at++;
+        copy_chunk(L.r[at], c);
+    }
+}
+
+// The frame of every tile (frames' tile ranges ascend), and the clip-list
+// counter cleared for the first pass.
+__global__ __launch_bounds__(256) void k_tile_frames(const DFrame* __restrict__ frames, uint32_t numFrames, uint32_t numTiles,
+                                                     uint32_t* __restrict__ tileFrame, uint32_t* __restrict__ clipCount) {
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t == 0) *clipCount = 0u;
+    if (t >= numTiles) return;
+    uint32_t lo = 0, hi = numFrames;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (frames[mid].tileBase <= t) lo = mid; else hi = mid;
+    }
+    tileFrame[t] = lo;
 }
 
 __global__ void k_fill_f32(float* __restrict__ p, size_t n) {
@@ -4438,6 +4489,7 @@ struct PFDjob {
     hipStream_t side = nullptr;           // the clip kernel beside k_setup<1> (default priority); may be null
     hipEvent_t fork = nullptr, join = nullptr;
     Arena* arena = nullptr;               // non-null: buffers come from the arena, never from hipMalloc
+    bool oneShot = false;                 // runs one frame after the other (pfdExecuteFrame)
     bool autoTiles = false;               // choose tile size and raster mode from the first counts
     uint64_t autoKey = 0;                 // one-shot job: shape of the last automatically configured
     uint32_t autoShift = 0, autoMode = 0; // frame and its choice (kept across job_reset)
@@ -4485,9 +4537,19 @@ struct PFDjob {
     DevBuf copyTable;                     // CopyRegions of the last download
     std::vector<CopyRegion> copies;       // the same on the host
     // Page-locked staging for copies from and to pageable host memory
-    // (staged_h2d / staged_d2h), made on first use.
+    // (staged_h2d / staged_d2h), made on first use; busy: its last transfer
+    // to the device may still be running.
     void* hstage[2] = { nullptr, nullptr };
     hipEvent_t hstageEv[2] = { nullptr, nullptr };
+    bool hstageBusy[2] = { false, false };
+    // Page-locked block of the small uploads (upload), made on first use: its
+    // first UP_HEAD bytes take what sizing runs read back, the rest is filled
+    // from `upUsed` and reused after a synchronisation.
+    uint8_t* upHost = nullptr;
+    uint8_t* upDev = nullptr;             // the same as kernels see it
+    size_t upCap = 0, upUsed = 0;
+    CopyList upList{};                    // regions not launched yet
+    bool clipDirty = false;               // a failed run may have left the clip-list counter off zero
 };
 
 namespace {
@@ -4641,22 +4703,27 @@ bool hstage_ready(PFDjob* J) {
     return true;
 }
 
-// Host -> device on the job's stream; returns with the host memory read.
+// Pageable host memory -> device, queued on the job's stream; returns with
+// the host memory read, the last transfers still running.
 hipError_t staged_h2d(PFDjob* J, void* dev, const void* host, size_t bytes) {
-    if (bytes < HSTAGE_CHUNK || host_pinned(host) || !hstage_ready(J)) {
+    // The staging chunks (4 MiB of page-locked memory) are made for a large
+    // copy, or for the job of one-shot frames, which uses them again.
+    const bool mayStage = J->hstage[0] || J->oneShot || bytes >= HSTAGE_CHUNK;
+    if (bytes < ((size_t)64 << 10) || !mayStage || host_pinned(host) || !hstage_ready(J)) {
         hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, J->stream);
         return e == hipSuccess ? hipStreamSynchronize(J->stream) : e;
     }
     hipError_t e = hipSuccess;
     for (size_t off = 0, i = 0; e == hipSuccess && off < bytes; off += HSTAGE_CHUNK, i++) {
         const size_t n = std::min(HSTAGE_CHUNK, bytes - off), b = i & 1;
-        if (i >= 2) e = hipEventSynchronize(J->hstageEv[b]);   // this chunk's last DMA is done
+        if (J->hstageBusy[b]) e = hipEventSynchronize(J->hstageEv[b]);   // this chunk's last DMA is done
         if (e != hipSuccess) break;
         CopyPool::get().copy(J->hstage[b], (const uint8_t*)host + off, n);
         e = hipMemcpyAsync((uint8_t*)dev + off, J->hstage[b], n, hipMemcpyHostToDevice, J->stream);
         if (e == hipSuccess) e = hipEventRecord(J->hstageEv[b], J->stream);
+        J->hstageBusy[b] = true;
     }
-    return e == hipSuccess ? hipStreamSynchronize(J->stream) : e;
+    return e;
 }
 
 // Device -> host after the work queued on the job's stream; returns with
@@ -4667,6 +4734,7 @@ hipError_t staged_d2h(PFDjob* J, void* host, const void* dev, size_t bytes) {
         return e == hipSuccess ? hipStreamSynchronize(J->stream) : e;
     }
     const size_t chunks = (bytes + HSTAGE_CHUNK - 1) / HSTAGE_CHUNK;
+    J->hstageBusy[0] = J->hstageBusy[1] = false;             // every chunk is waited for below
     auto issue = [&](size_t i) -> hipError_t {
         const size_t off = i * HSTAGE_CHUNK, n = std::min(HSTAGE_CHUNK, bytes - off);
         hipError_t ee = hipMemcpyAsync(J->hstage[i & 1], (const uint8_t*)dev + off, n, hipMemcpyDeviceToHost, J->stream);
@@ -4745,12 +4813,66 @@ struct Downloads {
     }
 };
 
-uint32_t read_total(PFDjob* J, int* rc) {
-    uint32_t v = 0;
-    hipError_t e = hipMemcpyAsync(&v, J->scanTotal.p, 4, hipMemcpyDeviceToHost, J->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(J->stream);
-    if (e != hipSuccess) { set_error("read_total", e); *rc = PFD_E_LAUNCH; }
-    return v;
+constexpr size_t UP_HEAD = 64, UP_SMALL = (size_t)128 << 10, UP_BLOCK = (size_t)512 << 10;
+
+// Launches the uploads added since the last one.
+int upload_flush(PFDjob* J) {
+    if (J->upList.n == 0) return PFD_OK;
+    hipLaunchKernelGGL(k_copy_list, dim3(std::min(J->upList.chunks, COPY_BLOCKS)), dim3(256), 0, J->stream, J->upList);
+    J->upList.n = J->upList.chunks = 0;
+    HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
+    return PFD_OK;
+}
+
+// The page-locked block of small uploads; false when there is none (a job
+// that may not allocate), and uploads go by copy commands.
+bool upload_ready(PFDjob* J) {
+    if (J->arena) return false;
+    if (J->upHost) return true;
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, UP_BLOCK, hipHostMallocDefault) != hipSuccess || hipHostGetDevicePointer(&d, h, 0) != hipSuccess || !d) {
+        (void)hipGetLastError();
+        if (h) (void)hipHostFree(h);
+        return false;
+    }
+    J->upHost = (uint8_t*)h;
+    J->upDev = (uint8_t*)d;
+    J->upCap = UP_BLOCK;
+    J->upUsed = UP_HEAD;
+    return true;
+}
+
+// Host -> device, in order with the job's stream.  Small sources are read
+// before it returns; page-locked ones above UP_SMALL are read by the next
+// upload_flush's kernel, and must stay as they are until the stream has been
+// synchronised.  Kernels that read `dev` are launched after upload_flush.
+int upload(PFDjob* J, void* dev, const void* host, size_t bytes) {
+    if (bytes == 0) return PFD_OK;
+    int rc;
+    const uint8_t* src = nullptr;
+    if (bytes <= UP_SMALL && upload_ready(J)) {
+        if (J->upUsed + bytes > J->upCap) {
+            if ((rc = upload_flush(J))) return rc;
+            HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
+            J->upUsed = UP_HEAD;
+        }
+        memcpy(J->upHost + J->upUsed, host, bytes);
+        src = J->upDev + J->upUsed;
+        J->upUsed += (bytes + 15) & ~(size_t)15;
+    } else if (bytes > UP_SMALL && !J->arena) {
+        src = host_mapped(const_cast<void*>(host), bytes);
+    }
+    const size_t c = (bytes + COPY_CHUNK - 1) / COPY_CHUNK;
+    if (src && c < 0x40000000u) {
+        if ((J->upList.n == COPY_INLINE || J->upList.chunks > 0x40000000u) && (rc = upload_flush(J))) return rc;
+        CopyRegion& r = J->upList.r[J->upList.n++];
+        r.src = src; r.dst = (uint8_t*)dev; r.bytes = bytes; r.firstChunk = J->upList.chunks;
+        J->upList.chunks += (uint32_t)c;
+        return PFD_OK;
+    }
+    if ((rc = upload_flush(J))) return rc;
+    HIP_TRY(staged_h2d(J, dev, host, bytes), PFD_E_LAUNCH);
+    return PFD_OK;
 }
 
 uint32_t grid_for(uint64_t n, uint32_t block) {
@@ -4977,14 +5099,14 @@ int run_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
     if ((rc = ensure(J, J->cnt, (size_t)n * 4 + 4)) || (rc = ensure(J, J->off, (size_t)n * 4 + 4))) return rc;
     if ((rc = ensure(J, J->blockRT, (size_t)nb * 4 + 4)) || (rc = ensure(J, J->blockPairs, (size_t)nb * 4 + 4))) return rc;
     if ((rc = ensure(J, J->scanTotal, 16))) return rc;
-    if ((rc = ensure(J, J->clipList, (size_t)n * 16 + 16)) || (rc = ensure(J, J->clipCount, 16))) return rc;
+    if ((rc = ensure(J, J->clipList, (size_t)n * 16 + 16))) return rc;
     if ((rc = ensure(J, J->clearSnap, J->frames.size() * 32))) return rc;
     const size_t fragSlots = (size_t)J->numTiles * 4;
     const size_t passIdx = (size_t)(&P - J->passes.data());
     if (discover) {
-        // Slots no wave writes (TS = 8 uses one of four) must read as zero.
         if ((rc = ensure(J, J->tileFrags, fragSlots * J->passes.size() * 4 + 4))) return rc;
-        hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(fragSlots, 256 * 8)), dim3(256), 0, J->stream,
+        if (n == 0 && !P.anyClear)                           // no raster kernel to write them
+            hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(fragSlots, 256 * 8)), dim3(256), 0, J->stream,
                            (uint32_t*)J->tileFrags.p + passIdx * fragSlots, (uint32_t)fragSlots, 0u);
     }
     if ((rc = ensure(J, J->tileBegin, (size_t)J->numTiles * 4 + 4)) || (rc = ensure(J, J->tileEnd, (size_t)J->numTiles * 4 + 4)))
@@ -5048,24 +5170,33 @@ int run_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
     }
     // Replays with few blocks leave the block sums raw for k_scan_local<true>.
     const bool fusedScan = !discover && nb <= 1024;
+    const bool readBack = discover && upload_ready(J);
     // Triangles to clip: counted once the pass is sized, estimated before.
     const uint32_t clip0 = discover ? n / 64 : P.numClip;
     for (;;) {
-        // Every pass leaves the clip-list counter at zero (k_tile_bounds, or
-        // the fill at its end); a discovering run clears it here as well.
-        if (discover)
+        // k_tile_frames clears the clip-list counter and every pass leaves it
+        // at zero (k_tile_bounds, or the fill at its end), unless a run failed.
+        if (discover && J->clipDirty)
             hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, J->stream, (uint32_t*)J->clipCount.p, 1u, 0u);
         hipLaunchKernelGGL((k_setup<0, false>), dim3(nb), dim3(256), 0, J->stream, sa);
         if (discover || P.numClip) launch_clip<0, false, VF_POS>(sa, clip0, J->stream);
         if (!fusedScan)
             hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(SCAN_THREADS), 0, J->stream,
-                               (uint32_t*)J->blockRT.p, (uint32_t*)J->blockPairs.p, nb, (uint32_t*)J->scanTotal.p);
+                               (uint32_t*)J->blockRT.p, (uint32_t*)J->blockPairs.p, nb, (uint32_t*)J->scanTotal.p,
+                               (const uint32_t*)J->clipCount.p, readBack ? (uint32_t*)J->upDev : nullptr);
         HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
         if (!discover) break;
         uint32_t tot[2] = {0, 0}, clipped = 0;
-        HIP_TRY(hipMemcpyAsync(tot, J->scanTotal.p, 8, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
-        HIP_TRY(hipMemcpyAsync(&clipped, J->clipCount.p, 4, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
+        if (!readBack) {
+            HIP_TRY(hipMemcpyAsync(tot, J->scanTotal.p, 8, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
+            HIP_TRY(hipMemcpyAsync(&clipped, J->clipCount.p, 4, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
+        }
         HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
+        if (readBack) {
+            const volatile uint32_t* back = (const volatile uint32_t*)J->upHost;
+            tot[0] = back[0]; tot[1] = back[1]; clipped = back[2];
+        }
+        J->clipDirty = false;
         P.numRT = tot[0];
         P.numPairs = tot[1];
         P.numClip = std::min(clipped, n);
@@ -5199,6 +5330,7 @@ int run_all(PFDjob* J, bool discover) {
             // clip list's) off zero; the next run rediscovers, which clears
             // them before use.
             for (auto& Q : J->passes) Q.sized = false;
+            J->clipDirty = true;
             return rc;
         }
     return 0;
@@ -5243,19 +5375,14 @@ void layout_tiles(PFDjob* J) {
 // Frame table, tile -> frame map and the per-pass tile descriptors; all
 // depend on the tile size, so they are uploaded again when it changes.
 int upload_frames_table(PFDjob* J) {
-    int rc = ensure(J, J->dFrames, J->frames.size() * sizeof(DFrame));
-    if (rc) return rc;
-    HIP_TRY(hipMemcpy(J->dFrames.p, J->frames.data(), J->frames.size() * sizeof(DFrame), hipMemcpyHostToDevice), PFD_E_LAUNCH);
-    std::vector<uint32_t> tf(J->numTiles ? J->numTiles : 1, 0u);
-    for (uint32_t f = 0; f < J->frames.size(); f++) {
-        const DFrame& F = J->frames[f];
-        for (uint32_t t = 0; t < F.tilesX * F.tilesY; t++) tf[F.tileBase + t] = f;
-    }
-    if ((rc = ensure(J, J->dTileFrame, tf.size() * 4))) return rc;
-    HIP_TRY(hipMemcpy(J->dTileFrame.p, tf.data(), tf.size() * 4, hipMemcpyHostToDevice), PFD_E_LAUNCH);
+    int rc;
     const size_t nf = J->frames.size();
+    if ((rc = ensure(J, J->dFrames, nf * sizeof(DFrame))) || (rc = ensure(J, J->clipCount, 16))
+        || (rc = ensure(J, J->dTileFrame, (size_t)(J->numTiles ? J->numTiles : 1) * 4))
+        || (rc = upload(J, J->dFrames.p, J->frames.data(), nf * sizeof(DFrame))))
+        return rc;
     std::vector<DTileFrame> d(J->passes.size() * nf);
-    memset(d.data(), 0, d.size() * sizeof(DTileFrame));
+    if (!d.empty()) memset(d.data(), 0, d.size() * sizeof(DTileFrame));
     for (size_t p = 0; p < J->passes.size(); p++) {
         const PassInfo& P = J->passes[p];
         for (size_t f = 0; f < nf; f++) {
@@ -5271,11 +5398,15 @@ int upload_frames_table(PFDjob* J) {
             t.clearDepth = sg.clearDepth;
         }
     }
-    if (d.empty()) return 0;
-    if ((rc = ensure(J, J->tileDescs, d.size() * sizeof(DTileFrame)))) return rc;
-    HIP_TRY(hipMemcpy(J->tileDescs.p, d.data(), d.size() * sizeof(DTileFrame), hipMemcpyHostToDevice), PFD_E_LAUNCH);
+    if (!d.empty() && ((rc = ensure(J, J->tileDescs, d.size() * sizeof(DTileFrame)))
+                       || (rc = upload(J, J->tileDescs.p, d.data(), d.size() * sizeof(DTileFrame)))))
+        return rc;
     for (size_t p = 0; p < J->passes.size(); p++)
         J->passes[p].dTileDesc = (const DTileFrame*)J->tileDescs.p + p * nf;
+    if ((rc = upload_flush(J))) return rc;
+    hipLaunchKernelGGL(k_tile_frames, dim3(grid_for(J->numTiles, 256)), dim3(256), 0, J->stream, (const DFrame*)J->dFrames.p,
+                       (uint32_t)nf, J->numTiles, (uint32_t*)J->dTileFrame.p, (uint32_t*)J->clipCount.p);
+    HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
     return 0;
 }
 
@@ -5403,6 +5534,9 @@ void job_reset(PFDjob* J) {
     J->diff = J->diffRan = false;
     J->numVertices = 0;
     J->paramTex = -1;
+    J->upUsed = UP_HEAD;
+    J->upList.n = J->upList.chunks = 0;
+    J->clipDirty = false;
     if (J->arena) {
         J->arena->used = 0;
         for_each_buf(J, [](DevBuf& b) { b = DevBuf(); });
@@ -5464,8 +5598,10 @@ const char* check_arrays(const PFFarrays& a, uint32_t prevEnd, uint32_t nt, uint
 // triangle streams, states and textures of all frames concatenated, render
 // targets, decoded pfDrawPixels images, points and lines (projected once),
 // and per pass its segments (one per frame at most) and pixel / point /
-// line operations.  The job's configuration must be set.
-int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
+// line operations.  The job's configuration must be set.  With `wait` the
+// frames' memory has been read when it returns; without, once the job's
+// stream has been synchronised.
+int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid, bool wait) {
     int rc = 0;
     hipError_t e = hipSuccess;
 
@@ -5559,8 +5695,8 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
     std::vector<RawImage> images;
     auto decode_images = [&](void) -> int {
         if (images.empty()) return 0;
-        e = hipStreamSynchronize(J->stream);                      // the stage's last images are decoded
-        if (e == hipSuccess) e = hipMemcpy(J->stage.p, hraw.data(), std::min(hraw.size(), J->stage.bytes), hipMemcpyHostToDevice);
+        // In order on the stream: the stage's last images are decoded before.
+        if ((rc = upload(J, J->stage.p, hraw.data(), std::min(hraw.size(), J->stage.bytes))) || (rc = upload_flush(J))) return rc;
         for (const RawImage& m : images) {
             if (e != hipSuccess) break;
             hipLaunchKernelGGL(k_decode_image, dim3((uint32_t)((m.texels + 255) / 256)), dim3(256), 0, J->stream,
@@ -5598,18 +5734,16 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
                 // Raw texels + 4 zero bytes (the getters' word reads run up
                 // to 3 bytes past the last texel), decoded to RGBA8.
                 const size_t rawBytes = texels * pff_source_texel_bytes(T.source);
-                e = staged_h2d(J, J->stage.p, T.pixels, rawBytes);
-                if (e == hipSuccess) e = hipMemsetAsync((uint8_t*)J->stage.p + rawBytes, 0, 4, J->stream);
-                if (e == hipSuccess) {
-                    hipLaunchKernelGGL(k_decode_texels, dim3((uint32_t)((texels + 255) / 256)), dim3(256), 0, J->stream,
-                                       (const uint8_t*)J->stage.p, texels, T.source, (uint32_t*)dst);
-                    e = hipGetLastError();
-                }
-                if (e == hipSuccess) e = hipStreamSynchronize(J->stream);   // the stage is reused
+                const uint32_t zero = 0u;
+                if ((rc = upload(J, J->stage.p, T.pixels, rawBytes))
+                    || (rc = upload(J, (uint8_t*)J->stage.p + rawBytes, &zero, 4)) || (rc = upload_flush(J)))
+                    return rc;
+                hipLaunchKernelGGL(k_decode_texels, dim3((uint32_t)((texels + 255) / 256)), dim3(256), 0, J->stream,
+                                   (const uint8_t*)J->stage.p, texels, T.source, (uint32_t*)dst);
+                e = hipGetLastError();
                 if (e != hipSuccess) { set_error("texture decode", e); return PFD_E_LAUNCH; }
             } else if (bytes) {
-                e = staged_h2d(J, dst, T.pixels, bytes);
-                if (e != hipSuccess) { set_error("texture upload", e); return PFD_E_LAUNCH; }
+                if ((rc = upload(J, dst, T.pixels, bytes))) return rc;
             }
             if (T.format == PFF_TEX_SOURCE) d.format = PFF_TEX_RGBA8;
             d.pixels = dst;
@@ -5641,18 +5775,25 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
         D.depth = (float*)((uint8_t*)J->targetPool.p + targetOff);
         targetOff += align256(npx * 4);
 
-        for (uint32_t k = 0; k < fr.numPoints; k++) {
-            PFFpoint q = fr.points[k];
-            if (q.state >= fr.numStates) PLAN_FAIL(PFD_E_INVALID, "bad point state");
-            q.state += stateBase;
-            hpts.push_back(q);
-        }
-        for (uint32_t k = 0; k < fr.numLines; k++) {
-            PFFline q = fr.lines[k];
-            if (q.state >= fr.numStates) PLAN_FAIL(PFD_E_INVALID, "bad line state");
-            q.state += stateBase;
-            if (k == 0) q.groupStart = 1u;             // groups never span frames
-            hlns.push_back(q);
+        // A single frame's points and lines go up as they are; several frames'
+        // are gathered with their states' places.
+        bool badPrim = false;
+        for (uint32_t k = 0; k < fr.numPoints; k++) badPrim |= fr.points[k].state >= fr.numStates;
+        if (badPrim) PLAN_FAIL(PFD_E_INVALID, "bad point state");
+        for (uint32_t k = 0; k < fr.numLines; k++) badPrim |= fr.lines[k].state >= fr.numStates;
+        if (badPrim) PLAN_FAIL(PFD_E_INVALID, "bad line state");
+        if (count > 1) {
+            for (uint32_t k = 0; k < fr.numPoints; k++) {
+                PFFpoint q = fr.points[k];
+                q.state += stateBase;
+                hpts.push_back(q);
+            }
+            for (uint32_t k = 0; k < fr.numLines; k++) {
+                PFFline q = fr.lines[k];
+                q.state += stateBase;
+                if (k == 0) q.groupStart = 1u;         // groups never span frames
+                hlns.push_back(q);
+            }
         }
         // Commands -> segments; the k-th segment of a frame runs in pass k.
         uint32_t segNo = 0;
@@ -5806,19 +5947,11 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
         lnBase += fr.numLines;
     }
 
-    if (!himg.empty()) {
-        e = hipMemcpy(J->pixPool.p, himg.data(), himg.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) { set_error("pixel image upload", e); return PFD_E_LAUNCH; }
-    }
+    if ((rc = upload(J, J->pixPool.p, himg.data(), himg.size()))) return rc;
     // Device copies of the inputs.
     auto up = [&](DevBuf& b, const void* h, size_t bytes) -> int {
-        int r = ensure(J, b, bytes ? bytes : 4);
-        if (r) return r;
-        if (bytes) {
-            hipError_t ee = hipMemcpy(b.p, h, bytes, hipMemcpyHostToDevice);
-            if (ee != hipSuccess) { set_error("upload", ee); return PFD_E_LAUNCH; }
-        }
-        return 0;
+        const int r = ensure(J, b, bytes ? bytes : 4);
+        return r ? r : upload(J, b.p, h, bytes);
     };
     const bool vidOn = wantVid && count == 1 && frames[0].tris.vertexId != nullptr;
     if (count == 1) {
@@ -5831,15 +5964,12 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
             || (rc = ensure(J, J->uv, T.texcoord ? n * 24 + 4 : 4)) || (rc = ensure(J, J->nrm, T.normal ? n * 36 + 4 : 4))
             || (vidOn && (rc = ensure(J, J->vid, n * 12 + 4))))
             return rc;
-        // Asynchronous on the job's stream: the host library records into
-        // page-locked memory, so these are DMA transfers queued back to back
-        // (no round trip each); the stream is synchronised at the end of
-        // this function, before the caller may touch the streams again.
+        // The host library records into page-locked memory, which the upload
+        // kernel reads in place.
         for_host_ranges(fr, [&](uint32_t b, uint32_t e2) {
             auto part = [&](DevBuf& d, const void* h, size_t per) {
-                if (e == hipSuccess && h)
-                    e = hipMemcpyAsync((uint8_t*)d.p + b * per, (const uint8_t*)h + b * per, (size_t)(e2 - b) * per,
-                                       hipMemcpyHostToDevice, J->stream);
+                if (!rc && h)
+                    rc = upload(J, (uint8_t*)d.p + b * per, (const uint8_t*)h + b * per, (size_t)(e2 - b) * per);
             };
             part(J->pos, T.position, 48);
             part(J->col, T.color, 12);
@@ -5848,7 +5978,7 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
             part(J->nrm, T.normal, 36);
             if (vidOn) part(J->vid, T.vertexId, 12);
         });
-        if (e != hipSuccess) { set_error("upload", e); return PFD_E_LAUNCH; }
+        if (rc) return rc;
     } else {
         std::vector<float> hpos((size_t)totalTris * 12);
         std::vector<uint32_t> hcol((size_t)totalTris * 3), hinfo(totalTris);
@@ -5879,13 +6009,12 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
             return rc;
         std::vector<DArrays> tab;
         tab.reserve(numDraws);
-        bool usedResident = false;
         uint8_t* dst = (uint8_t*)J->arrPool.p;
         uint32_t tb = 0, sb = 0, cum = 0;
         auto put = [&](const void* h, size_t bytes) -> const uint8_t* {
             if (!h) return nullptr;
             uint8_t* d = dst;
-            if (bytes && e == hipSuccess) e = hipMemcpy(d, h, bytes, hipMemcpyHostToDevice);
+            if (!rc) rc = upload(J, d, h, bytes);
             dst += align256(bytes);
             return d;
         };
@@ -5907,7 +6036,6 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
                     d.nrm = at(a.normal);
                     d.uv = at(a.texcoord);
                     d.col = at(a.colors);
-                    usedResident = true;
                 } else {
                     d.pos = put(a.position, n * a.posSize * elem_bytes(a.posType));
                     d.nrm = put(a.normal, n * 3 * elem_bytes(a.nrmType));
@@ -5937,47 +6065,19 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
             tb += fr.tris.count;
             sb += fr.numStates;
         }
-        if (e == hipSuccess) e = hipMemcpy(J->arrTable.p, tab.data(), tab.size() * sizeof(DArrays), hipMemcpyHostToDevice);
-        if (e != hipSuccess) { set_error("array draw upload", e); return PFD_E_LAUNCH; }
-        if (arrTris) {
-            hipLaunchKernelGGL(k_deindex, dim3((uint32_t)((arrTris + 255) / 256)), dim3(256), 0, J->stream,
-                               (const DArrays*)J->arrTable.p, numDraws, (uint32_t)arrTris, (float4*)J->pos.p,
-                               (uint32_t*)J->col.p, anyUV ? (float2*)J->uv.p : nullptr,
-                               anyNrm ? (float*)J->nrm.p : nullptr, (uint32_t*)J->info.p,
-                               vidOn ? (uint32_t*)J->vid.p : nullptr);
-            HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
-        }
-        // Resident copies belong to their lists, which may go once the
-        // frame has been handed over: read them before returning.
-        if (usedResident) HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
+        if (rc || (rc = upload(J, J->arrTable.p, tab.data(), tab.size() * sizeof(DArrays)))) return rc;
     }
     if ((rc = up(J->states, hstates.data(), hstates.size() * sizeof(PFFstate)))
         || (rc = up(J->texTable, htex.data(), htex.size() * sizeof(DTex))))
         return rc;
-    if (!hpts.empty()) {
-        // Points are projected once; every replay reads the projections.
-        if ((rc = up(J->points, hpts.data(), hpts.size() * sizeof(PFFpoint)))
-            || (rc = ensure(J, J->pointScr, hpts.size() * sizeof(DPointScr))))
-            return rc;
-        const uint32_t np = (uint32_t)hpts.size();
-        hipLaunchKernelGGL(k_point_setup, dim3((np + 255) / 256), dim3(256), 0, J->stream, (const PFFpoint*)J->points.p,
-                           np, (const PFFstate*)J->states.p, (DPointScr*)J->pointScr.p);
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(J->stream);
-        if (e != hipSuccess) { set_error("point setup", e); return PFD_E_LAUNCH; }
-    }
-    if (!hlns.empty()) {
-        // Lines are projected and clipped once; every replay reads them.
-        if ((rc = up(J->lines, hlns.data(), hlns.size() * sizeof(PFFline)))
-            || (rc = ensure(J, J->lineScr, hlns.size() * sizeof(DLineScr))))
-            return rc;
-        const uint32_t nl = (uint32_t)hlns.size();
-        hipLaunchKernelGGL(k_line_setup, dim3((nl + 255) / 256), dim3(256), 0, J->stream, (const PFFline*)J->lines.p,
-                           nl, (const PFFstate*)J->states.p, (DLineScr*)J->lineScr.p);
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(J->stream);
-        if (e != hipSuccess) { set_error("line setup", e); return PFD_E_LAUNCH; }
-    }
+    // Points and lines are projected (and lines clipped) once; every replay
+    // reads the projections.
+    if (ptBase && ((rc = up(J->points, count == 1 ? frames[0].points : hpts.data(), (size_t)ptBase * sizeof(PFFpoint)))
+                   || (rc = ensure(J, J->pointScr, (size_t)ptBase * sizeof(DPointScr)))))
+        return rc;
+    if (lnBase && ((rc = up(J->lines, count == 1 ? frames[0].lines : hlns.data(), (size_t)lnBase * sizeof(PFFline)))
+                   || (rc = ensure(J, J->lineScr, (size_t)lnBase * sizeof(DLineScr)))))
+        return rc;
     // Per-pass tables, all passes in one buffer (one copy).
     std::vector<size_t> offs;
     size_t tabBytes = 0;
@@ -6061,6 +6161,23 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
         J->dPixOps = put(hpix);
         if ((rc = up(J->passTab, tab.data(), tabBytes))) return rc;
     }
+    layout_tiles(J);
+    if ((rc = upload_frames_table(J))) return rc;             // and everything added before
+    if (arrTris) {
+        hipLaunchKernelGGL(k_deindex, dim3((uint32_t)((arrTris + 255) / 256)), dim3(256), 0, J->stream,
+                           (const DArrays*)J->arrTable.p, numDraws, (uint32_t)arrTris, (float4*)J->pos.p,
+                           (uint32_t*)J->col.p, anyUV ? (float2*)J->uv.p : nullptr,
+                           anyNrm ? (float*)J->nrm.p : nullptr, (uint32_t*)J->info.p,
+                           vidOn ? (uint32_t*)J->vid.p : nullptr);
+        HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
+    }
+    if (ptBase)
+        hipLaunchKernelGGL(k_point_setup, dim3((ptBase + 255) / 256), dim3(256), 0, J->stream, (const PFFpoint*)J->points.p,
+                           ptBase, (const PFFstate*)J->states.p, (DPointScr*)J->pointScr.p);
+    if (lnBase)
+        hipLaunchKernelGGL(k_line_setup, dim3((lnBase + 255) / 256), dim3(256), 0, J->stream, (const PFFline*)J->lines.p,
+                           lnBase, (const PFFstate*)J->states.p, (DLineScr*)J->lineScr.p);
+    HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
     if (markWords) {
         hipLaunchKernelGGL(k_fill_u32, dim3(std::min(4096u, grid_for(markWords, 256 * 4))), dim3(256), 0, J->stream,
                            (uint32_t*)J->runMarks.p, (uint32_t)markWords, 0u);
@@ -6075,12 +6192,26 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid) {
             }
         HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
     }
-    layout_tiles(J);
-    if ((rc = upload_frames_table(J))) return rc;
-    // The caller may change its streams once this returns: the asynchronous
-    // uploads above must have read them.
-    HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
+    // The caller may change its streams once this returns, and lists their
+    // resident copies: the work above must have read them.
+    if (wait) HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
     return PFD_OK;
+}
+
+// Host render targets -> device, queued on the job's stream.  A frame whose
+// first command is a clear needs only pixels 0..7 (all other pixels are
+// overwritten or copy pixel 0).
+int upload_targets(PFDjob* J) {
+    int rc = 0;
+    for (size_t f = 0; f < J->frames.size(); f++) {
+        const PFFframe& fr = J->src[f];
+        const size_t npx = (size_t)fr.width * fr.height;
+        const size_t n = J->leadClear[f] ? (npx < 8 ? npx : 8) : npx;
+        if ((rc = upload(J, J->frames[f].depth, fr.depth, n * 4))
+            || (rc = upload(J, J->frames[f].color, fr.color, n * pff_target_bytes(fr.target))))
+            return rc;
+    }
+    return upload_flush(J);
 }
 
 #undef PLAN_FAIL
@@ -6098,7 +6229,7 @@ int pfdJobCreate(const PFFframe* frames, uint32_t count, const PFDconfig* cfg, P
     if ((rc = job_shell(&J, true))) return rc;
     J->cfg = cfg ? *cfg : g_defaultCfg;
     J->tileShift = (J->cfg.tileShift >= 3 && J->cfg.tileShift <= 6) ? J->cfg.tileShift : 3;
-    if ((rc = job_plan(J, frames, count, false))) { pfdJobDestroy(J); return rc; }
+    if ((rc = job_plan(J, frames, count, false, true))) { pfdJobDestroy(J); return rc; }
     *out = J;
     return PFD_OK;
 }
@@ -6119,18 +6250,10 @@ int pfdJobSetConfig(PFDjob* J, const PFDconfig* cfg) {
     return PFD_OK;
 }
 
-// Host render targets -> device.  A frame whose first command is a clear
-// needs only pixels 0..7 (all other pixels are overwritten or copy pixel 0).
 int pfdJobUploadTargets(PFDjob* J) {
     if (!J) return PFD_E_INVALID;
-    for (size_t f = 0; f < J->frames.size(); f++) {
-        const PFFframe& fr = J->src[f];
-        size_t npx = (size_t)fr.width * fr.height;
-        bool leadClear = J->leadClear[f] != 0;
-        size_t n = leadClear ? (npx < 8 ? npx : 8) : npx;
-        HIP_TRY(hipMemcpyAsync(J->frames[f].depth, fr.depth, n * 4, hipMemcpyHostToDevice, J->stream), PFD_E_LAUNCH);
-        HIP_TRY(staged_h2d(J, J->frames[f].color, fr.color, n * pff_target_bytes(fr.target)), PFD_E_LAUNCH);
-    }
+    int rc = upload_targets(J);
+    if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
     return PFD_OK;
 }
@@ -6341,6 +6464,8 @@ void pfdHostFree(void* p) {
     else free(h);
 }
 
+void pfdHostCopy(void* dst, const void* src, size_t bytes) { CopyPool::get().copy(dst, src, bytes); }
+
 struct PFDresident {
     void*  p;
     size_t bytes;
@@ -6383,6 +6508,7 @@ void pfdJobDestroy(PFDjob* J) {
         if (J->hstage[i]) (void)hipHostFree(J->hstage[i]);
         if (J->hstageEv[i]) (void)hipEventDestroy(J->hstageEv[i]);
     }
+    if (J->upHost) (void)hipHostFree(J->upHost);
     if (J->fork) (void)hipEventDestroy(J->fork);
     if (J->join) (void)hipEventDestroy(J->join);
     if (J->side) (void)hipStreamDestroy(J->side);
@@ -6422,9 +6548,9 @@ int run_one_shot(PFDjob* J, const PFFframe* frames, uint32_t count) {
         J->cfg.rasterMode = J->autoMode;
     }
     const bool choosing = J->autoTiles;
-    int rc = job_plan(J, frames, count, false);
-    if (!rc && !(rc = pfdJobUploadTargets(J)) && !(rc = run_all(J, true)) && !(rc = pfdJobSync(J)))
-        rc = pfdJobDownload(J);
+    int rc = job_plan(J, frames, count, false, false);
+    if (!rc && !(rc = upload_targets(J)) && !(rc = run_all(J, true))) rc = pfdJobDownload(J);
+    if (rc) (void)hipStreamSynchronize(J->stream);            // nothing still reads the frames
     if (!rc && choosing) {
         J->autoKey = shape;
         J->autoShift = J->tileShift;
@@ -6452,6 +6578,7 @@ int pfdExecuteFrames(const PFFframe* frames, uint32_t count) {
     std::unique_lock<std::mutex> lk(g_oneShotLock, std::try_to_lock);
     if (lk.owns_lock()) {
         if (!g_oneShot && (rc = job_shell(&g_oneShot, true))) return rc;
+        g_oneShot->oneShot = true;
         job_reset(g_oneShot);
         return run_one_shot(g_oneShot, frames, count);
     }
@@ -6551,7 +6678,7 @@ int pfdDiffCreate(const PFFframe* frame, PFDjob** out) {
     J->tileShift = (J->cfg.tileShift >= 3 && J->cfg.tileShift <= 6) ? J->cfg.tileShift : 3;
     // The corners' colour-array indices (host-recorded or formed from array
     // draws) address the colour parameters.
-    if ((rc = job_plan(J, frame, 1, true))) { pfdJobDestroy(J); return rc; }
+    if ((rc = job_plan(J, frame, 1, true, true))) { pfdJobDestroy(J); return rc; }
     J->diff = true;
     const size_t npx = (size_t)frame->width * frame->height;
     if ((rc = ensure(J, J->winner, npx * 4)) || (rc = ensure(J, J->image, npx * 16)) || (rc = ensure(J, J->dImage, npx * 16))) {

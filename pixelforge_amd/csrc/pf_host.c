@@ -122,6 +122,8 @@ typedef struct {                       /* the frame being recorded */
     PFFline*   lns;      size_t nlns, caplns;
     PFFarrays* arr;      size_t narr, caparr;   /* array draws; element copies owned */
     uint8_t*   arrOwned;  size_t capowned;      /* per array draw: 1 if its block is owned */
+    uint8_t*   blk;       size_t capblk, nblk;  /* pfdHostAlloc memory of the array draws' blocks */
+    size_t     wantblk;                         /* bytes of this frame's blocks that did not fit */
     ListStore** stores;  size_t nstores, capstores;   /* lists called, one reference each */
     int        anyTex, anyLight, anyVid;
 } Rec;
@@ -326,12 +328,40 @@ static int grow(void** p, size_t* cap, size_t need, size_t elem)
 
 static void store_release(ListStore* st);
 
+/* Array draws' blocks beyond this many bytes a frame stay on the heap. */
+#define MAX_REC_BLOCK ((size_t)64 << 20)
+
+/* A block of an array draw's elements, from the frame's page-locked memory
+ * (uploads then read it in place) or, where that is full, from the heap
+ * (*owned: to be freed with the frame). */
+static void* rec_block(Rec* r, size_t bytes, int* owned)
+{
+    const size_t n = (bytes + 63) & ~(size_t)63;
+    *owned = 0;
+    if (r->blk && n <= r->capblk - r->nblk) {
+        void* p = r->blk + r->nblk;
+        r->nblk += n;
+        return p;
+    }
+    r->wantblk += n;
+    *owned = 1;
+    return malloc(bytes);
+}
+
 static void rec_reset(Rec* r)
 {
     for (size_t i = 0; i < r->npix; i++) free((void*)r->pix[i].pixels);
     for (size_t i = 0; i < r->narr; i++)
         if (r->arrOwned[i]) free((void*)r->arr[i].position);             /* one block per draw */
     r->narr = 0;
+    if (r->wantblk && r->nblk + r->wantblk <= MAX_REC_BLOCK) {
+        /* Room for the next frame of this size. */
+        const size_t bytes = r->nblk + r->wantblk + (r->nblk + r->wantblk) / 4;
+        pfdHostFree(r->blk);
+        r->blk = (uint8_t*)pfdHostAlloc(bytes);
+        r->capblk = r->blk ? bytes : 0;
+    }
+    r->nblk = r->wantblk = 0;
     for (size_t i = 0; i < r->nstores; i++) store_release(r->stores[i]);
     r->nstores = 0;
     r->npix = 0;
@@ -353,8 +383,9 @@ static void rec_free(Rec* r)
     free(r->arrOwned);
     free(r->arr);
     free(r->pix);
-    free(r->pts);
-    free(r->lns);
+    pfdHostFree(r->pts);
+    pfdHostFree(r->lns);
+    pfdHostFree(r->blk);
     pfdHostFree(r->pos); pfdHostFree(r->col); pfdHostFree(r->uv); pfdHostFree(r->nrm);
     pfdHostFree(r->info); pfdHostFree(r->vid);
     free(r->states); free(r->texs); free(r->texKeys); free(r->cmds);
@@ -558,6 +589,18 @@ static int host_grow(void** p, size_t used, size_t bytes)
     return 1;
 }
 
+/* Grows an array of points or lines, kept in pfdHostAlloc memory as the
+ * triangle streams are. */
+static int prim_grow(void** p, size_t* cap, size_t need, size_t elem)
+{
+    if (need <= *cap) return 1;
+    size_t nc = *cap ? *cap : 256;
+    while (nc < need) nc *= 2;
+    if (!host_grow(p, *cap * elem, nc * elem)) return 0;
+    *cap = nc;
+    return 1;
+}
+
 /* Grows the triangle streams to hold at least `need` triangles.  They live
  * in pfdHostAlloc memory (page-locked with a GPU), from which a frame's
  * upload is a direct DMA transfer. */
@@ -653,7 +696,7 @@ static void emit_point(Ctx* c, const Vert* v)
     int si = current_state(c);
     if (si < 0) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
     Rec* r = &c->rec;
-    if (!grow((void**)&r->pts, &r->cappts, r->npts + 1, sizeof(PFFpoint))) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
+    if (!prim_grow((void**)&r->pts, &r->cappts, r->npts + 1, sizeof(PFFpoint))) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
     PFFpoint* p = &r->pts[r->npts];
     memcpy(p->position, v->position, 16);
     p->color = pack(v->color);
@@ -681,7 +724,7 @@ static void emit_line(Ctx* c, const Vert* a, const Vert* b, int groupStart)
     int si = current_state(c);
     if (si < 0) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
     Rec* r = &c->rec;
-    if (!grow((void**)&r->lns, &r->caplns, r->nlns + 1, sizeof(PFFline))) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
+    if (!prim_grow((void**)&r->lns, &r->caplns, r->nlns + 1, sizeof(PFFline))) { set_err(PF_ERROR_OUT_OF_MEMORY); return; }
     PFFline* l = &r->lns[r->nlns];
     memcpy(l->position[0], a->position, 16);
     memcpy(l->position[1], b->position, 16);
@@ -1772,24 +1815,28 @@ static int record_array_draw(Ctx* c, PFdrawmode mode, PFsizei count, PFdatatype 
     const size_t cb = useC ? (size_t)c->aCol.size * type_bytes(c->aCol.type) : 0;
 #define ALIGN16(x) (((x) + 15) & ~(size_t)15)
     const size_t total = ALIGN16(n * pb) + ALIGN16(n * nb) + ALIGN16(n * tb) + ALIGN16(n * cb) + (size_t)count * isz + 16;
-    uint8_t* blk = (uint8_t*)malloc(total);
+    /* The target first: a frame for another one is executed before this
+     * draw's block is taken from the frame's memory. */
+    if (!ensure_target(c)) { set_err(PF_INVALID_OPERATION); pfEnd(); return 1; }
+    int owned;
+    uint8_t* blk = (uint8_t*)rec_block(&c->rec, total, &owned);
     if (!blk) { set_err(PF_ERROR_OUT_OF_MEMORY); pfEnd(); return 1; }
-    PFFarrays* d = push_array_draw(c, mode, (uint32_t)count, tris, groups, passes, blk, 1);
+    PFFarrays* d = push_array_draw(c, mode, (uint32_t)count, tris, groups, passes, blk, owned);
     if (!d) { pfEnd(); return 1; }
     uint8_t* q = blk;
-    memcpy(q, (const uint8_t*)c->aPos.buffer + lo * pb, n * pb);
+    pfdHostCopy(q, (const uint8_t*)c->aPos.buffer + lo * pb, n * pb);
     d->posSize = c->aPos.size; d->posType = (uint32_t)c->aPos.type;
     q += ALIGN16(n * pb);
-    if (useN) { memcpy(q, (const uint8_t*)c->aNrm.buffer + lo * nb, n * nb); d->normal = q; d->nrmType = (uint32_t)c->aNrm.type; }
+    if (useN) { pfdHostCopy(q, (const uint8_t*)c->aNrm.buffer + lo * nb, n * nb); d->normal = q; d->nrmType = (uint32_t)c->aNrm.type; }
     q += ALIGN16(n * nb);
-    if (useUV) { memcpy(q, (const uint8_t*)c->aUV.buffer + lo * tb, n * tb); d->texcoord = q; d->uvType = (uint32_t)c->aUV.type; }
+    if (useUV) { pfdHostCopy(q, (const uint8_t*)c->aUV.buffer + lo * tb, n * tb); d->texcoord = q; d->uvType = (uint32_t)c->aUV.type; }
     q += ALIGN16(n * tb);
     if (useC) {
-        memcpy(q, (const uint8_t*)c->aCol.buffer + lo * cb, n * cb);
+        pfdHostCopy(q, (const uint8_t*)c->aCol.buffer + lo * cb, n * cb);
         d->colors = q; d->colSize = c->aCol.size; d->colType = (uint32_t)c->aCol.type;
     }
     q += ALIGN16(n * cb);
-    if (indices) { memcpy(q, indices, (size_t)count * isz); d->indices = q; d->idxType = (uint32_t)itype; }
+    if (indices) { pfdHostCopy(q, indices, (size_t)count * isz); d->indices = q; d->idxType = (uint32_t)itype; }
 #undef ALIGN16
     d->elementBase = (uint32_t)lo;
     d->numElements = (uint32_t)n;
