@@ -1,0 +1,50 @@
+"""Gradients gathered per 16x16 block before they go to memory, at the sizes
+where the gathering can go wrong: more texels or vertices in a block than
+its tables hold, every pixel of a block on one triangle and few texels,
+target sides that leave part of a block empty, all light slots in use.  The
+adjoint is compared with the FP64 oracle of the same frame: relative error
+<= 1e-3 per gradient, by norm and by element, the suite's bound for FP32
+sums."""
+import numpy as np
+import pytest
+
+import pixelforge_amd as pf
+from diffscene import Scene, oracle_job, params_of, target_of
+
+pytestmark = pytest.mark.gpu
+
+REL = 1e-3
+
+CASES = {
+    "minified_texels": dict(width=48, height=48, nx=4, nz=4, tex=(256, 256), seed=21),       # ~1000 texels a block
+    "tiny_triangles": dict(width=40, height=40, nx=60, nz=60, tex=(16, 16), seed=22),         # ~600 vertices a block
+    "one_triangle_a_block": dict(width=64, height=64, nx=1, nz=1, tex=(2, 2), seed=23),
+    "one_texel": dict(width=33, height=31, nx=2, nz=2, tex=(1, 1), seed=24),
+    "ragged_nearest": dict(width=53, height=17, nx=9, nz=5, tex=(33, 7), filt=pf.PF_NEAREST, seed=25),
+    "few_pixels": dict(width=3, height=2, nx=2, nz=2, tex=(4, 4), seed=26),
+    "four_lights": dict(width=50, height=30, nx=6, nz=6, lights=4, attenuation=True, spot=True, seed=27),
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_gathered_gradients_match_fp64(case):
+    if pf.lib().pfdInit() != 0:
+        pytest.fail("no GPU: " + pf.lib().pfdLastError().decode())
+    s = Scene(**CASES[case])
+    try:
+        job = oracle_job(s)
+        s.rerecord()
+        p64 = params_of(s)
+        p32 = [a.astype(np.float32) for a in p64]
+        img64 = job.forward(*p64)
+        img = s.gpu_forward(*p32)
+        assert np.abs(img - img64).max() <= 2e-5
+        d = (2.0 * (img64 - target_of(s, job))).astype(np.float32)
+        g = s.gpu_backward(*p32, d)
+        g64 = job.backward(*p64, d.astype(np.float64))
+        for name, a, b in zip(("texels", "colors", "ldiff", "lspec"), g, g64):
+            a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+            assert np.linalg.norm(a - b) <= REL * np.linalg.norm(b), name
+            assert np.abs(a - b).max() <= REL * np.abs(b).max(), name
+    finally:
+        s.close()
