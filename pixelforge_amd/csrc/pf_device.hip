@@ -2003,10 +2003,12 @@ struct RasterArgs {
 //
 // Each wave owns one 8x8 block of a tile (one pixel per lane; colour and
 // depth stay in VGPRs from the fused clear / load to the single write-back)
-// and walks the tile's pair list in batches of 32: the 32 lanes fetch 32
-// list entries and their raster-triangle records in one round trip, keep
-// the ones whose bbox meets the block and stage them, compacted and still in
-// list order, in the wave's LDS.  Each staged triangle is then tested
+// and walks the tile's pair list 64 entries at a time (32 where a lane stages
+// whole lit records at once): the lanes fetch the entries and their
+// raster-triangle records in one round trip, keep the ones whose bbox meets
+// the block (and, in the HIZ instances, that are not behind all its pixels)
+// and stage them, compacted and still in list order, up to 32 at once, in the
+// wave's LDS.  Each staged triangle is then tested
 // against the block (edge functions per lane, ballot).  Two ways to shade:
 //   packed   (mode 0): covered (triangle, pixel) fragments are queued in LDS
 //            with a per-pixel chain in submission order; when 64 are queued
@@ -3711,7 +3713,8 @@ __device__ __forceinline__ void walk_run(const RunMarks& m, uint32_t tile, uint3
 // instructions each).  Each operation was a pass of its own before: a frame
 // of 100 rects and 32 images of 32x32 over a fogged 800x600 scene ran 133
 // of them, 3.2 us each behind six launches of an empty triangle pass, an
-// upload and a synchronisation (whole call 14.1 -> 0.49 ms).
+// upload and a synchronisation (whole call 14.1 -> 0.49 ms when the runs came
+// in, 0.33 since a frame's uploads go in one launch).
 __global__ __launch_bounds__(256) void k_pixel_runs(const DPixRun* __restrict__ runs, const DPixOp* __restrict__ ops) {
     const DPixRun o = runs[blockIdx.y];
     if (blockIdx.x >= o.tilesX * o.tilesY) return;
