@@ -2263,11 +2263,15 @@ constexpr uint32_t REC_HIDDEN = 0x80000000u;
 // GEQUAL test, `dep` the largest negated depth.  Leading chunks q0..q3 and
 // z[2] of a META_NOWRAP record.  `full`: the triangle covers the whole block.
 //
-// A fragment's depth is rcp_x86(s), s = sum z_k b_k with b_k = w_k / sum w:
+// A fragment's depth is rcp_x86(s), s = sum z_k b_k with b_k = w_k wInvSum:
 // s is affine over the block, so its exact values there lie between its
-// extremes at the corners, and at covered pixels (b_k >= 0, sum 1) also
-// between the extremes of z_k.  What the float evaluation here and per pixel
-// adds is below 2^-20 of the largest sum of |z_k b_k| at a corner; 2^-19 is
+// extremes at the corners.  At covered pixels (b_k >= 0) they lie also between
+// the extremes of z_k where the b_k add up to 1.  They need not: wInvSum
+// inverts the sum of the weights taken mod 2^32, which can wrap though no w_k
+// does; the b_k then add up to at least 2 off 1 (a sum of magnitude below
+// 3 * 2^31 over one of at most 2^31 that differs from it by a multiple of
+// 2^32).  What the float evaluation here and per pixel adds is below 2^-20 of
+// the largest sum of |z_k b_k| at a corner; 2^-19 is
 // allowed.  rcp_x86 is within 2^-11 of 1 / s while neither is subnormal
 // (tests/test_rcp_table.py); 2^-10 is allowed, and an interval of s that
 // reaches 0 (the depth may be anything) or leaves the normal range hides
@@ -2279,7 +2283,7 @@ __device__ __forceinline__ bool hidden_behind(uint4 q0, uint4 q1, uint4 q2, uint
     const int32_t eC[3] = { (int32_t)q1.z, (int32_t)q1.w, (int32_t)q2.x };
     const float inv = __uint_as_float(q3.y);
     const float z[3] = { sign * __uint_as_float(q3.z), sign * __uint_as_float(q3.w), sign * __uint_as_float(z2) };
-    float s = 0.0f, gx = 0.0f, gy = 0.0f, mag = 0.0f;
+    float s = 0.0f, gx = 0.0f, gy = 0.0f, mag = 0.0f, one = 0.0f;
     int32_t low = 0;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -2287,13 +2291,16 @@ __device__ __forceinline__ bool hidden_behind(uint4 q0, uint4 q1, uint4 q2, uint
         low |= w + min(dx, 0) + min(dy, 0);
         const float b = (float)w * inv, bx = (float)dx * inv, by = (float)dy * inv;
         s += z[k] * b;
+        one += b;
         gx += z[k] * bx;
         gy += z[k] * by;
         mag += fabsf(z[k]) * (fabsf(b) + fabsf(bx) + fabsf(by) + 1.0f);
     }
     full = low >= 0;
     const float err = mag * 0x1p-19f;
-    const float zl = fminf(z[0], fminf(z[1], z[2])), zh = fmaxf(z[0], fmaxf(z[1], z[2]));
+    const float inf = __builtin_inff();
+    const bool sums = fabsf(one - 1.0f) < 0.5f;    // the b_k add up to 1
+    const float zl = sums ? fminf(z[0], fminf(z[1], z[2])) : -inf, zh = sums ? fmaxf(z[0], fmaxf(z[1], z[2])) : inf;
     const float lo = fmaxf(s + fminf(gx, 0.0f) + fminf(gy, 0.0f), zl) - err;
     const float hi = fminf(s + fmaxf(gx, 0.0f) + fmaxf(gy, 0.0f), zh) + err;
     const float r = __builtin_amdgcn_rcpf(hi);

@@ -111,3 +111,109 @@ def test_layers_match_oracle(name, target):
         L.pfMakeCurrent(ctx)
         L.pfDeleteContext(ctx)
         L.pfMakeCurrent(None)
+
+
+def _jobs_match_oracle(record, size, what):
+    """`record`: makes a context with a recorded frame, and its buffer.  The
+    frame at every tile size and raster mode, a sizing run and a replay each,
+    against the oracle's."""
+    L = pf.lib()
+    with OracleExecutor() as ex:
+        ctx, want = record()
+        L.pfFinish()
+        samples = ex.fragments
+        L.pfDeleteContext(ctx)
+    ctx, got = record()
+    L.pfxSetExecutor(C.cast(L.pfdCaptureExecutor, C.c_void_p), None)
+    try:
+        L.pfFinish()
+    finally:
+        L.pfxSetExecutor(None, None)
+    cap = pf.Captured(L.pfdTakeCapturedJob(), [], [], [])
+    try:
+        depth = cap.targets()[0][1]
+        snap = got.copy(), depth.copy()
+        for shift, mode in [(3, 0), (3, 1), (4, 2), (4, 0), (4, 1), (5, 0), (5, 1), (6, 0), (6, 1)]:
+            print(f"{what} tile {1 << shift} mode {mode}", flush=True)
+            cfg = pf.PFDconfig()
+            cfg.tileShift, cfg.rasterMode = shift, mode
+            assert L.pfdJobSetConfig(cap.job, C.byref(cfg)) == 0
+            for run in range(2):
+                got[:], depth[:] = snap
+                assert L.pfdJobUploadTargets(cap.job) == 0
+                assert L.pfdJobLaunch(cap.job) == 0 and L.pfdJobSync(cap.job) == 0 and L.pfdJobDownload(cap.job) == 0
+                bad = np.count_nonzero(got != want)
+                assert bad == 0, f"{what} tile {1 << shift} mode {mode} run {run}: {bad} bytes differ"
+                st = pf.PFDstats()
+                assert L.pfdJobStats(cap.job, C.byref(st)) == 0
+                assert int(st.fragments) == samples
+    finally:
+        cap.close()
+        L.pfMakeCurrent(ctx)
+        L.pfDeleteContext(ctx)
+        L.pfMakeCurrent(None)
+
+
+def _weights(corners, w, h):
+    """Edge values of a triangle of screen corners at pixel (0, 0), its
+    largest magnitude of one within 128 pixels of the target, and their sum."""
+    (x1, y1), (x2, y2), (x3, y3) = [(int(x), int(y)) for x, y in corners]
+    a = (y3 - y2, y1 - y3, y2 - y1)
+    b = (x2 - x3, x3 - x1, x1 - x2)
+    c = [-(ox * a[k] + oy * b[k]) for k, (ox, oy) in enumerate(((x2, y2), (x3, y3), (x1, y1)))]
+    far = max(abs(a[k] * x + b[k] * y + c[k]) for k in range(3) for x in (-128, w + 128) for y in (-128, h + 128))
+    return c, far, sum(c)
+
+
+def _record_wrapping(seed, size, func):
+    """Seventy layers, then triangles around the target so large that the sum
+    of a pixel's three weights leaves 32 bits where no weight does: their
+    barycentric coordinates do not add up to one."""
+    L = pf.lib()
+    w, h = size
+    buf = np.full((w * h + 16) * 4, 9, np.uint8)
+    ctx = C.c_void_p(L.pfCreateContext(buf.ctypes.data, w, h, 7, 0))
+    L.pfMakeCurrent(ctx)
+    rng = np.random.default_rng(seed)
+    sign = -1.0 if func >= GREATER else 1.0
+    for matrix in (1, 0):
+        L.pfMatrixMode(matrix)
+        L.pfLoadIdentity()
+    L.pfDisable(0x10)
+    L.pfEnable(0x8)
+    L.pfClearDepth(*_f(sign * 3e38))
+    L.pfClear(3)
+    L.pfDepthFunc(func)
+
+    def triangle(corners, z):
+        L.pfBegin(2)
+        L.pfColor4ub(*rng.integers(0, 256, 4).tolist())
+        for (x, y), zk in zip(corners, z):
+            # Half a pixel off the edge of the truncation to whole pixels.
+            L.pfVertex3f(*_f(2.0 * (x + 0.5 * np.sign(x)) / (w - 1) - 1.0, 1.0 - 2.0 * (y + 0.5 * np.sign(y)) / (h - 1), zk))
+        L.pfEnd()
+
+    for k in range(70):
+        d = sign * (1.0 + (70 - k) * 0.01)                        # the layers end at a depth of 1.01
+        triangle([(-9, -9), (-9, 9 * h), (9 * w, -9)], [1.0 / d] * 3)
+    wrapped = 0
+    for _ in range(40):
+        s = rng.uniform(22000, 27000)
+        corners = [(-s, -s), (-s, 2 * s), (2 * s, -s)] + rng.uniform(-0.02, 0.02, (3, 2)) * s
+        if rng.random() < 0.5:
+            corners = corners[[0, 2, 1]]
+        corners = np.trunc(corners)
+        _, far, total = _weights(corners, w, h)
+        wrapped += far < 2**31 - 2**24 and abs(total) > 2**31 + 2**24
+        # Behind the layers if the coordinates added up to one.
+        z = sign * rng.uniform(0.3, 0.75) * (1.0 if rng.random() < 0.3 else rng.uniform(0.8, 1.25, 3)) * np.ones(3)
+        triangle(corners, z)
+    assert wrapped >= 20
+    assert L.pfGetError() == 0
+    return ctx, buf
+
+
+@pytest.mark.parametrize("func", [LESS, LEQUAL, GREATER, GEQUAL])
+def test_triangles_whose_weights_wrap_match_oracle(func):
+    for seed, size in ((1, (101, 75)), (2, (33, 140))):
+        _jobs_match_oracle(lambda: _record_wrapping(seed, size, func), size, f"function {func} size {size}")
