@@ -60,7 +60,8 @@ typedef struct {
     uint32_t numTiles;
     uint32_t tileShift;
     uint64_t deviceBytes;      /* device memory held by the job               */
-    uint32_t maxTileList;      /* longest per-tile pair list (last pass)      */
+    uint32_t maxTileList;      /* longest per-tile pair list (last pass; 0 if
+                                  it draws no triangles)                     */
     uint32_t busyTiles;        /* tiles with a non-empty list (last pass)     */
     uint32_t clippedTriangles; /* recorded triangles that needed clipping     */
     uint32_t reserved;

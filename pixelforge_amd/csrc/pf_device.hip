@@ -6458,7 +6458,8 @@ int pfdJobStats(PFDjob* J, PFDstats* st) {
     size_t bytes = 0;
     for_each_buf(J, [&](DevBuf& b) { bytes += b.bytes; });
     st->deviceBytes = bytes;
-    if (J->tileBegin.p && J->numTiles) {
+    // A pass without triangles leaves the lists as they are (run_pass).
+    if (J->tileBegin.p && J->numTiles && !J->passes.empty() && J->passes.back().numPassTris) {
         std::vector<uint32_t> b(J->numTiles), e(J->numTiles);
         HIP_TRY(hipMemcpy(b.data(), J->tileBegin.p, (size_t)J->numTiles * 4, hipMemcpyDeviceToHost), PFD_E_LAUNCH);
         HIP_TRY(hipMemcpy(e.data(), J->tileEnd.p, (size_t)J->numTiles * 4, hipMemcpyDeviceToHost), PFD_E_LAUNCH);
