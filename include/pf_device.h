@@ -118,7 +118,8 @@ int pfdExecuteFrameNoAlloc(const PFFframe* frame);
  * ignored). */
 void* pfdHostAlloc(size_t bytes);
 void  pfdHostFree(void* p);
-/* memcpy between host buffers, split over a few threads from 256 KiB on. */
+/* memcpy between host buffers, split over a few threads from 256 KiB on where
+ * they are free (one copy has them at a time; a child of fork() has none). */
 void  pfdHostCopy(void* dst, const void* src, size_t bytes);
 
 /* Device copies of host bytes that outlive frames (no reference

@@ -32,6 +32,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 #include <stddef.h>
 #include <math.h>
 #include <vector>
@@ -4707,9 +4708,14 @@ class CopyPool {
         static CopyPool* pool = new CopyPool();
         return *pool;
     }
+    // The threads do not exist in a child of fork(), which copies by itself;
+    // so does a caller that finds them at work for another (contexts on
+    // several threads recording 11 MB each: 0.10 ms, 0.36 with four of them
+    // waiting for each other).
     void copy(void* dst, const void* src, size_t bytes) {
-        if (workers_.empty() || bytes < ((size_t)256 << 10)) { memcpy(dst, src, bytes); return; }
-        std::lock_guard<std::mutex> one(callLock_);          // one parallel copy at a time
+        if (workers_.empty() || bytes < ((size_t)256 << 10) || getpid() != owner_) { memcpy(dst, src, bytes); return; }
+        std::unique_lock<std::mutex> one(callLock_, std::try_to_lock);
+        if (!one.owns_lock()) { memcpy(dst, src, bytes); return; }
         const size_t parts = workers_.size() + 1;
         const size_t per = ((bytes + parts - 1) / parts + 63) & ~(size_t)63;
         {
@@ -4747,6 +4753,7 @@ class CopyPool {
             if (--pending_ == 0) done_.notify_one();
         }
     }
+    const pid_t owner_ = getpid();
     std::vector<std::thread> workers_;
     std::mutex callLock_, m_;
     std::condition_variable cv_, done_;
