@@ -93,3 +93,47 @@ def test_uploads_match_oracle(count, verts, tex, typ):
     for k, (a, b) in enumerate(zip(want, got)):
         assert len(np.unique(a)) > 50
         assert np.array_equal(a, b), f"image {k}: {np.count_nonzero(a != b)} pixels differ"
+
+
+def _images(sizes, seed):
+    L = pf.lib()
+    w, h = 260, 200
+    rng = np.random.default_rng(seed)
+    buf = np.zeros(w * h + 16, np.uint32)
+    ctx = C.c_void_p(L.pfCreateContext(buf.ctypes.data, w, h, 7, 0))
+    L.pfMakeCurrent(ctx)
+    L.pfDisable(0x10)
+    out = []
+    for _ in range(2):
+        L.pfClear(3)
+        for k, (iw, ih, fmt, typ, bpp) in enumerate(sizes):
+            px = rng.integers(0, 256, iw * ih * bpp).astype(np.uint8)
+            L.pfRasterPos3f(*_f(-1 + 0.1 * k, 1 - 0.1 * k, 0.0))
+            L.pfPixelZoom(*_f(0.7, 0.7))
+            L.pfDrawPixels(iw, ih, fmt, typ, C.c_void_p(px.ctypes.data))
+            px[:] = 3                                 # the frame holds its own copy
+        L.pfFinish()
+        out.append(buf[:w * h].copy())
+    assert L.pfGetError() == 0
+    L.pfDeleteContext(ctx)
+    L.pfMakeCurrent(None)
+    return out
+
+
+@pytest.mark.parametrize("sizes", [
+    [(181, 181, 7, 0, 4), (182, 181, 7, 0, 4), (9, 7, 7, 0, 4)],                       # 131044, 131768 bytes
+    [(3, 3, 6, 0, 3), (211, 207, 6, 0, 3), (211, 208, 6, 0, 3), (256, 256, 7, 4, 2)],  # 131031, 131664, 131072
+    [(640, 480, 7, 0, 4), (333, 400, 6, 0, 3), (5, 4, 9, 3, 2), (700, 500, 4, 0, 1), (16, 16, 7, 0, 4),
+     (120, 90, 6, 2, 2), (1500, 900, 8, 0, 3), (40, 40, 7, 0, 4)]],
+    ids=["rgba8", "raw", "mixed"])
+def test_images_around_the_gathered_size_match_oracle(sizes):
+    """pfDrawPixels images on both sides of the size up to which a frame's
+    images are gathered, raw and RGBA8 ones in turn."""
+    print(sizes, flush=True)
+    with OracleExecutor():
+        want = _images(sizes, 4)
+    pf.lib().pfxSetExecutor(None, None)
+    got = _images(sizes, 4)
+    for k, (a, b) in enumerate(zip(want, got)):
+        assert len(np.unique(a)) > 50
+        assert np.array_equal(a, b), f"frame {k}: {np.count_nonzero(a != b)} pixels differ"
