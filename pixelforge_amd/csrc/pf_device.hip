@@ -3535,7 +3535,7 @@ __device__ __forceinline__ uint32_t tgt_set_scalar(uint32_t kind, uint32_t c) {
 }
 
 struct DPixOp {
-    uint32_t  kind;               // 0 pfDrawPixels, 1 pfFogProcess, 2 pfRect*
+    uint32_t  kind;               // 0 an image, 1 pfFogProcess, 2 a plain rect (plain_rect)
     const uint32_t* texels;       // kind 0: w*h RGBA8
     uint32_t  color;              // kind 2: the fill colour
     uint32_t  w, h;
@@ -3774,8 +3774,10 @@ __global__ __launch_bounds__(256) void k_pixel_runs(const DPixRun* __restrict__ 
                     uint32_t at = f2u32_x86(v * (float)(s.h - 1u)) * s.w + f2u32_x86(u * (float)(s.w - 1u));
                     if (at >= n) at = n - 1u;
                     src = s.texels[at];
-                    d = s.zPos;
-                    dirtyZ = true;
+                    if (!(s.flags & PFF_PIXELS_RECT)) {           // pfRect writes no depth
+                        d = s.zPos;
+                        dirtyZ = true;
+                    }
                     blend = (s.flags & PFF_BLEND) != 0u;
                 }
             }
@@ -5658,6 +5660,14 @@ size_t elem_bytes(uint32_t type) {
     }
 }
 
+// A pfRect* fill as the host library records it: one RGBA8 colour, neither
+// tested nor blended.  Any other image with the rect flag is an image that
+// writes no depth.
+bool plain_rect(const PFFpixels& op) {
+    return (op.flags & PFF_PIXELS_RECT) && !(op.flags & (PFF_DEPTH_TEST | PFF_BLEND)) && op.width == 1u && op.height == 1u
+        && op.source == PFF_SOURCE(7, 0);
+}
+
 // Checks an array draw of a frame with `nt` triangles and `ns` states
 // against the rules of PFFarrays; returns a message or null.
 const char* check_arrays(const PFFarrays& a, uint32_t prevEnd, uint32_t nt, uint32_t ns) {
@@ -5755,7 +5765,7 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid, bo
             const PFFpixels& op = fr.pixelOps[cmd.first];
             const uint32_t bpp = pff_source_texel_bytes(op.source);
             if (bpp == 0u || op.width == 0u || op.height == 0u || !op.pixels) PLAN_FAIL(PFD_E_INVALID, "bad pixel image");
-            if (op.flags & PFF_PIXELS_RECT) continue;             // its colour goes into the operation
+            if (plain_rect(op)) continue;                         // its colour goes into the operation
             const size_t texels = (size_t)op.width * op.height;
             pixBytes += align256(texels * 4);
             if (op.source == PFF_SOURCE(7, 0)) {
@@ -6009,7 +6019,7 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid, bo
                 d.xMin = op.xMin; d.yMin = op.yMin; d.xMax = op.xMax; d.yMax = op.yMax;
                 d.zPos = op.zPos; d.invXLen = op.invXLen; d.invYLen = op.invYLen;
                 d.flags = op.flags; d.depthFunc = op.depthFunc; d.blendMode = op.blendMode;
-                if (op.flags & PFF_PIXELS_RECT) {
+                if (plain_rect(op)) {
                     d.kind = 2u;
                     memcpy(&d.color, op.pixels, 4);
                     add_pixel_op(d);
