@@ -4863,11 +4863,13 @@ uint8_t* host_mapped(void* p, size_t bytes) {
 // and then run; returns with the host memory written.  Page-locked
 // destinations are written by k_copy_out in one launch (a job that may not
 // allocate copies them one by one), the others through staged_d2h meanwhile.
+// Destinations that overlap (frames of one job given the same buffer) are
+// copied one by one in the order added, so that the last one's bytes stand.
 struct Downloads {
     PFDjob* J;
-    struct Staged { void* host; const void* dev; size_t bytes; };
+    struct Item { void* host; const void* dev; size_t bytes; uint8_t* mapped; };
+    std::vector<Item> items;
     std::vector<CopyRegion> regions;
-    std::vector<Staged> staged;
     uint32_t chunks = 0;
     explicit Downloads(PFDjob* job) : J(job) {}
     void add(void* host, const void* dev, size_t bytes) {
@@ -4876,29 +4878,57 @@ struct Downloads {
         // against 1191 us).
         uint8_t* m = J->arena || bytes > ((size_t)24 << 20) ? nullptr : host_mapped(host, bytes);
         const size_t c = (bytes + COPY_CHUNK - 1) / COPY_CHUNK;
-        if (!m || c > 0x7FFFFFFFu - chunks) { staged.push_back({ host, dev, bytes }); return; }
+        if (c > 0x7FFFFFFFu - chunks) m = nullptr;
+        items.push_back({ host, dev, bytes, m });
+        if (!m) return;
         CopyRegion r;
         memset(&r, 0, sizeof r);
         r.src = (const uint8_t*)dev; r.dst = m; r.bytes = bytes; r.firstChunk = chunks;
         chunks += (uint32_t)c;
         regions.push_back(r);
     }
+    bool overlap() const {
+        std::vector<std::pair<uintptr_t, size_t>> at;
+        at.reserve(items.size());
+        for (const Item& t : items) at.emplace_back((uintptr_t)t.host, t.bytes);
+        std::sort(at.begin(), at.end());
+        for (size_t i = 1; i < at.size(); i++)
+            if (at[i].first - at[i - 1].first < at[i - 1].second) return true;
+        return false;
+    }
+    // J->copies is what the device's table holds.
+    bool tabled() const {
+        return J->copies.size() == regions.size()
+            && memcmp(J->copies.data(), regions.data(), regions.size() * sizeof(CopyRegion)) == 0;
+    }
+    int upload_table() {
+        const size_t bytes = regions.size() * sizeof(CopyRegion);
+        const int rc = ensure(J, J->copyTable, bytes);
+        if (rc) return rc;
+        J->copies.swap(regions);
+        HIP_TRY(hipMemcpyAsync(J->copyTable.p, J->copies.data(), bytes, hipMemcpyHostToDevice, J->stream), PFD_E_LAUNCH);
+        return PFD_OK;
+    }
     int run() {
-        if (!regions.empty()) {
-            const size_t bytes = regions.size() * sizeof(CopyRegion);
-            int rc = ensure(J, J->copyTable, bytes);
+        bool kernel = !regions.empty();
+        if (kernel) {
+            // Regions in the table did not overlap when they came there.
+            const bool same = tabled();
+            kernel = (same && items.size() == regions.size()) || !overlap();
+            const int rc = kernel && !same ? upload_table() : 0;
             if (rc) return rc;
-            if (J->copies.size() != regions.size() || memcmp(J->copies.data(), regions.data(), bytes) != 0) {
-                J->copies.swap(regions);
-                HIP_TRY(hipMemcpyAsync(J->copyTable.p, J->copies.data(), bytes, hipMemcpyHostToDevice, J->stream), PFD_E_LAUNCH);
-            }
+        }
+        if (kernel) {
             hipLaunchKernelGGL(k_copy_out, dim3(std::min(chunks, COPY_BLOCKS)), dim3(256), 0, J->stream,
                                (const CopyRegion*)J->copyTable.p, (uint32_t)J->copies.size(), chunks);
             HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
         }
-        for (const Staged& t : staged) {
-            if (host_pinned(t.host)) HIP_TRY(hipMemcpyAsync(t.host, t.dev, t.bytes, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
-            else HIP_TRY(staged_d2h(J, t.host, t.dev, t.bytes), PFD_E_LAUNCH);
+        for (const Item& t : items) {
+            if (kernel && t.mapped) continue;
+            if (t.mapped || host_pinned(t.host))
+                HIP_TRY(hipMemcpyAsync(t.host, t.dev, t.bytes, hipMemcpyDeviceToHost, J->stream), PFD_E_LAUNCH);
+            else
+                HIP_TRY(staged_d2h(J, t.host, t.dev, t.bytes), PFD_E_LAUNCH);
         }
         HIP_TRY(hipStreamSynchronize(J->stream), PFD_E_LAUNCH);
         return PFD_OK;
