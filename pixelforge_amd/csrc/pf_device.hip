@@ -4896,17 +4896,20 @@ struct Downloads {
             if (at[i].first - at[i - 1].first < at[i - 1].second) return true;
         return false;
     }
-    // J->copies is what the device's table holds.
+    // J->copies is what the device's table holds, empty while that is not
+    // known.
     bool tabled() const {
         return J->copies.size() == regions.size()
             && memcmp(J->copies.data(), regions.data(), regions.size() * sizeof(CopyRegion)) == 0;
     }
     int upload_table() {
         const size_t bytes = regions.size() * sizeof(CopyRegion);
+        J->copies.clear();
         const int rc = ensure(J, J->copyTable, bytes);
         if (rc) return rc;
         J->copies.swap(regions);
-        HIP_TRY(hipMemcpyAsync(J->copyTable.p, J->copies.data(), bytes, hipMemcpyHostToDevice, J->stream), PFD_E_LAUNCH);
+        const hipError_t e = hipMemcpyAsync(J->copyTable.p, J->copies.data(), bytes, hipMemcpyHostToDevice, J->stream);
+        if (e != hipSuccess) { J->copies.clear(); set_error("download table", e); return PFD_E_LAUNCH; }
         return PFD_OK;
     }
     int run() {
