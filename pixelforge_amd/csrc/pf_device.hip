@@ -5216,7 +5216,7 @@ int finish_pass(PFDjob* J, PassInfo& P, hipEvent_t* ev) {
 // are read back (synchronising) and scratch buffers are sized; otherwise
 // the sizes of the previous run are used and nothing synchronises, so the
 // pass can be captured in a graph.
-int run_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
+int issue_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
     int rc = 0;
     if (P.numPassTris == 0 && P.segs.empty()) return 0;
     const uint32_t n = P.numPassTris;
@@ -5447,17 +5447,22 @@ int run_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
     return finish_pass(J, P, ev);
 }
 
+// issue_pass for every caller.  A pass that stopped part-way may leave device
+// counters (the clip list's) off zero; the next run discovers again, which
+// clears them before use.
+int run_pass(PFDjob* J, PassInfo& P, bool discover, hipEvent_t* ev) {
+    const int rc = issue_pass(J, P, discover, ev);
+    if (rc) {
+        for (auto& Q : J->passes) Q.sized = false;
+        J->clipDirty = true;
+    }
+    return rc;
+}
+
 int run_all(PFDjob* J, bool discover) {
     int rc = 0;
     for (auto& P : J->passes)
-        if ((rc = run_pass(J, P, discover || !P.sized, nullptr))) {
-            // A run that stopped part-way may leave device counters (the
-            // clip list's) off zero; the next run rediscovers, which clears
-            // them before use.
-            for (auto& Q : J->passes) Q.sized = false;
-            J->clipDirty = true;
-            return rc;
-        }
+        if ((rc = run_pass(J, P, discover || !P.sized, nullptr))) return rc;
     return 0;
 }
 

@@ -40,6 +40,35 @@ PRELUDE = """
     assert L.pfdInit() == 0, L.pfdLastError()
 """
 
+RUN_TIMED = PRELUDE + """
+    params = pf.scene(kind=pf.RANDOM_3D, width=160, height=120, ntris=4000, seed=12, depthFunc=pf.PF_LEQUAL)
+    with OracleExecutor():
+        want, _, err = pf.render(params, pf.LIB_PATH)
+    assert err == 0
+    failed = 0
+    for n in range(60):
+        cap = pf.capture(params)
+        snap = cap.snapshot()
+        cap.restore(snap)
+        t = pf.PFDtimes()
+        shim.shim_arm(n)
+        rc = L.pfdJobRunTimed(cap.job, C.byref(t))
+        shim.shim_arm(-1)
+        failed += rc != 0
+        for run in range(2):
+            cap.restore(snap)
+            assert L.pfdJobLaunch(cap.job) == 0 and L.pfdJobSync(cap.job) == 0 and L.pfdJobDownload(cap.job) == 0
+            got = cap.images()[0][:want.size].reshape(want.shape)
+            assert np.array_equal(got, want), (n, rc, run, np.count_nonzero(got != want))
+        st = pf.PFDstats()
+        assert L.pfdJobStats(cap.job, C.byref(st)) == 0 and st.clippedTriangles > 0
+        cap.close()
+        print("timed run, allocation", n, "rc", rc, flush=True)
+        if rc == 0:
+            break
+    assert 10 < failed < 60
+"""
+
 BATCH = PRELUDE + """
     def context(w, h, seed):
         px = np.zeros(w * h + 16, np.uint32)
@@ -88,7 +117,7 @@ BATCH = PRELUDE + """
 """
 
 
-@pytest.mark.parametrize("script", [BATCH], ids=["batch"])
+@pytest.mark.parametrize("script", [RUN_TIMED, BATCH], ids=["timed_run", "batch"])
 def test_the_call_after_a_failed_allocation_draws_whole(script, tmp_path):
     src, so = tmp_path / "shim.c", tmp_path / "shim.so"
     src.write_text(SHIM)
