@@ -2756,28 +2756,30 @@ __device__ __forceinline__ int32_t clamp_off(const DTex& t, int32_t off) {
 // Texel offsets and weights of one lookup, with the index maps of
 // sample_tex (sampler.h:202-334) and the same out-of-texture clamp.
 __device__ __forceinline__ void tex_taps(const DTex& t, float u, float v, Taps& tp) {
+    // Stored once at the end: stores in both branches were merged into one
+    // through a chosen address, which kept the taps in scratch memory.
     const uint32_t w = t.w;
-    if (t.filter == 0) {
-        int32_t x = wrap_coord(t.wrap, u, t.w), y = wrap_coord(t.wrap, v, t.h);
-        tp.n = 1;
-        tp.off[0] = clamp_off(t, (int32_t)((uint32_t)y * w + (uint32_t)x));
-        tp.w[0] = 1.0f;
-        return;
+    const int32_t x0 = wrap_coord(t.wrap, u, t.w), y0 = wrap_coord(t.wrap, v, t.h);
+    int32_t off1 = 0, off2 = 0, off3 = 0, n = 1;
+    float w0 = 1.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
+    if (t.filter != 0) {
+        float tx = rcp_int_rn(t.w), ty = rcp_int_rn(t.h);   // texture sides are at most 65535
+        int32_t x1 = wrap_coord(t.wrap, u + tx, t.w), y1 = wrap_coord(t.wrap, v + ty, t.h);
+        float fx = clamp_ps(u * (float)t.w - (float)x0, 0.0f, 1.0f);
+        float fy = clamp_ps(v * (float)t.h - (float)y0, 0.0f, 1.0f);
+        n = 4;
+        off1 = clamp_off(t, (int32_t)((uint32_t)y0 * w + (uint32_t)x1));
+        off2 = clamp_off(t, (int32_t)((uint32_t)y1 * w + (uint32_t)x0));
+        off3 = clamp_off(t, (int32_t)((uint32_t)y1 * w + (uint32_t)x1));
+        w0 = (1.0f - fx) * (1.0f - fy);
+        w1 = fx * (1.0f - fy);
+        w2 = (1.0f - fx) * fy;
+        w3 = fx * fy;
     }
-    float tx = rcp_int_rn(t.w), ty = rcp_int_rn(t.h);   // texture sides are at most 65535
-    int32_t x0 = wrap_coord(t.wrap, u, t.w), y0 = wrap_coord(t.wrap, v, t.h);
-    int32_t x1 = wrap_coord(t.wrap, u + tx, t.w), y1 = wrap_coord(t.wrap, v + ty, t.h);
-    float fx = clamp_ps(u * (float)t.w - (float)x0, 0.0f, 1.0f);
-    float fy = clamp_ps(v * (float)t.h - (float)y0, 0.0f, 1.0f);
-    tp.n = 4;
+    tp.n = n;
     tp.off[0] = clamp_off(t, (int32_t)((uint32_t)y0 * w + (uint32_t)x0));
-    tp.off[1] = clamp_off(t, (int32_t)((uint32_t)y0 * w + (uint32_t)x1));
-    tp.off[2] = clamp_off(t, (int32_t)((uint32_t)y1 * w + (uint32_t)x0));
-    tp.off[3] = clamp_off(t, (int32_t)((uint32_t)y1 * w + (uint32_t)x1));
-    tp.w[0] = (1.0f - fx) * (1.0f - fy);
-    tp.w[1] = fx * (1.0f - fy);
-    tp.w[2] = (1.0f - fx) * fy;
-    tp.w[3] = fx * fy;
+    tp.off[1] = off1; tp.off[2] = off2; tp.off[3] = off3;
+    tp.w[0] = w0; tp.w[1] = w1; tp.w[2] = w2; tp.w[3] = w3;
 }
 
 __device__ __forceinline__ float4 texel_f(const DiffArgs& A, const DTex& t, bool param, int32_t off) {
@@ -3944,6 +3946,18 @@ struct __attribute__((aligned(16))) DLineScr {
 };
 static_assert(sizeof(DLineScr) == 64, "DLineScr layout");
 
+// A record by four 16-byte loads, field by field: a plain copy kept the fields
+// that nothing reads before the record goes to LDS in scratch memory.
+__device__ __forceinline__ void load_line(const DLineScr* p, DLineScr& t) {
+    const uint4* q = reinterpret_cast<const uint4*>(p);
+    const uint4 a = q[0], b = q[1], c = q[2], d = q[3];
+    t.s1[0] = __uint_as_float(a.x); t.s1[1] = __uint_as_float(a.y);
+    t.s2[0] = __uint_as_float(a.z); t.s2[1] = __uint_as_float(a.w);
+    t.z1 = __uint_as_float(b.x); t.z2 = __uint_as_float(b.y); t.c1 = b.z; t.c2 = b.w;
+    t.flags = c.x; t.wAxis = c.y; t.bx0 = (int32_t)c.z; t.by0 = (int32_t)c.w;
+    t.bx1 = (int32_t)d.x; t.by1 = (int32_t)d.y; t.dec = (int32_t)d.z; t.inv = __uint_as_float(d.w);
+}
+
 // Fixed-point slope of a thin line (ints X1..Y2) along its longer axis, and
 // the reciprocal of its length there.
 __device__ __forceinline__ void line_slope(int32_t X1, int32_t Y1, int32_t X2, int32_t Y2, int32_t& dec, float& inv) {
@@ -4226,7 +4240,7 @@ __global__ __launch_bounds__(256) void k_lines(const DLnOp* __restrict__ ops, co
     };
     walk_run<DLineScr>(o.marks, blockIdx.x, o.last - o.first,
         [&](uint32_t i, DLineScr& t) {
-            t = run[i];
+            load_line(&run[i], t);
             return line_meets_tile(t, W, x0, y0);
         },
         [&](const DLineScr& s) {
