@@ -4070,7 +4070,8 @@ __global__ __launch_bounds__(256) void k_line_setup(const PFFline* __restrict__ 
             o.z1 = h1[2];
             o.z2 = h2[2];
             o.flags = st.flags & (PFF_DEPTH_TEST | PFF_BLEND);
-            o.flags |= (st.depthFunc & 7u) << 8 | (st.blendMode & 7u) << 12;
+            // Three bits each: every value above 7 acts as 7 does.
+            o.flags |= min(st.depthFunc, 7u) << 8 | min(st.blendMode, 7u) << 12;
             const int32_t x1 = cvtt_i32(o.s1[0]), y1 = cvtt_i32(o.s1[1]), x2 = cvtt_i32(o.s2[0]), y2 = cvtt_i32(o.s2[1]);
             int32_t w = 0, axis = 0;
             if (l.width > 1.5f) {
