@@ -3938,13 +3938,23 @@ struct __attribute__((aligned(16))) DLineScr {
     float    z1, z2;
     uint32_t c1, c2;
     uint32_t flags;               // PFF_DEPTH_TEST | PFF_BLEND; depth function << 8, blend mode << 12;
-                                  // 0x80000000 inactive; 0x40000000 thick
+                                  // 0x80000000 inactive; 0x40000000 thick; LINE_FAR
     uint32_t wAxis;               // thick copies: 1..w each side (low 16 bits), along axis (bit 16: 0 x, 1 y)
     int32_t  bx0, by0, bx1, by1;  // pixel bounds of every copy
     int32_t  dec;                 // of the centre line (line_step): fixed-point slope and
     float    inv;                 // 1 / length along the longer axis
 };
 static_assert(sizeof(DLineScr) == 64, "DLineScr layout");
+
+// DLineScr::flags of a line whose bounds and line_span may not hold its pixels:
+// k * dec in line_step passes 2^31 on longer ones (and the slope's rounding
+// leaves line_span's margin), and coordinates may be so large that their own
+// rounding counts.  NaN: far.
+constexpr uint32_t LINE_FAR = 0x20000000u;
+__device__ __forceinline__ bool line_far(const DLineScr& t) {
+    const float far = fmaxf(fmaxf(fabsf(t.s1[0]), fabsf(t.s1[1])), fmaxf(fabsf(t.s2[0]), fabsf(t.s2[1])));
+    return !(far < 1e6f && fabsf(t.s2[0] - t.s1[0]) < 32768.0f && fabsf(t.s2[1] - t.s1[1]) < 32768.0f);
+}
 
 // A record by four 16-byte loads, field by field: a plain copy kept the fields
 // that nothing reads before the record goes to LDS in scratch memory.
@@ -4072,6 +4082,7 @@ __global__ __launch_bounds__(256) void k_line_setup(const PFFline* __restrict__ 
             o.flags = st.flags & (PFF_DEPTH_TEST | PFF_BLEND);
             // Three bits each: every value above 7 acts as 7 does.
             o.flags |= min(st.depthFunc, 7u) << 8 | min(st.blendMode, 7u) << 12;
+            if (line_far(o)) o.flags |= LINE_FAR;
             const int32_t x1 = cvtt_i32(o.s1[0]), y1 = cvtt_i32(o.s1[1]), x2 = cvtt_i32(o.s2[0]), y2 = cvtt_i32(o.s2[1]);
             int32_t w = 0, axis = 0;
             if (l.width > 1.5f) {
@@ -4109,9 +4120,11 @@ struct DLnOp {
     RunMarks  marks;
 };
 
-// Whether any copy of the line leaves the target's columns: its pixels are
+// Whether any copy of the line may leave the target's columns: its pixels are
 // addressed y * W + x, so those land in a neighbouring row.
-__device__ __forceinline__ bool line_wraps(const DLineScr& t, int32_t W) { return t.bx0 < 0 || t.bx1 >= W; }
+__device__ __forceinline__ bool line_wraps(const DLineScr& t, int32_t W) {
+    return t.bx0 < 0 || t.bx1 >= W || (t.flags & LINE_FAR);
+}
 
 // Bounds of the shorter-axis coordinates of every copy of a line over the
 // tile's longer-axis interval [a, a + 15].  A pixel of the line lies within
@@ -4133,21 +4146,12 @@ __device__ __forceinline__ bool line_y_major(const DLineScr& t) {
     return fabsf(t.s2[1] - t.s1[1]) > fabsf(t.s2[0] - t.s1[0]);
 }
 
-// Whether line_span bounds the line: longer ones may leave its margin (the
-// slope's rounding), and so may coordinates whose own rounding counts.
-// NaN: no.
-__device__ __forceinline__ bool line_has_span(const DLineScr& t) {
-    const float far = fmaxf(fmaxf(fabsf(t.s1[0]), fabsf(t.s1[1])), fmaxf(fabsf(t.s2[0]), fabsf(t.s2[1])));
-    return far < 1e6f && fabsf(t.s2[0] - t.s1[0]) < 32768.0f && fabsf(t.s2[1] - t.s1[1]) < 32768.0f;
-}
-
 // Whether a line can touch the 16x16 tile at (x0, y0): its bounds, and for
 // lines that do not wrap the tile's distance from it.
 __device__ __forceinline__ bool line_meets_tile(const DLineScr& t, int32_t W, int32_t x0, int32_t y0) {
     if ((t.flags & 0x80000000u) || t.by1 < y0 - 1 || t.by0 > y0 + 16) return false;
     if (line_wraps(t, W)) return true;
     if (t.bx1 < x0 || t.bx0 > x0 + 15) return false;
-    if (!line_has_span(t)) return true;
     const bool yMajor = line_y_major(t);
     const float q0 = (float)(yMajor ? x0 : y0);
     float lo, hi;
@@ -4173,10 +4177,9 @@ __global__ __launch_bounds__(256) void k_line_mark(const DLnOp* __restrict__ ops
     const int32_t tx0 = x0 >> 4, tx1 = x1 >> 4, ty0 = y0 >> 4, ty1 = y1 >> 4;
     const bool yMajor = line_y_major(t);
     const int32_t p0 = yMajor ? ty0 : tx0, p1 = yMajor ? ty1 : tx1, q0 = yMajor ? tx0 : ty0, q1 = yMajor ? tx1 : ty1;
-    const bool spans = !wraps && line_has_span(t);
     for (int32_t p = p0; p <= p1; p++) {
         int32_t a = q0, b = q1;
-        if (spans) {
+        if (!wraps) {
             float lo, hi;
             line_span(t, yMajor, (float)(p * 16), lo, hi);
             a = max(a, cvtt_i32(fmaxf(lo, 0.0f)) >> 4);

@@ -1,4 +1,5 @@
-"""Lines at the ends of their ranges, against the oracle: states whose depth
+"""Lines at the ends of their ranges, against the oracle: ones longer than the
+16-bit slope reaches, whose steps leave their bounds, and states whose depth
 function and blend mode are no enum values."""
 import ctypes as C
 
@@ -6,11 +7,56 @@ import numpy as np
 import pytest
 
 import pixelforge_amd as pf
-from conftest import _oracle
+from conftest import OracleExecutor, _oracle
 from frames import on_frame
-from test_gpu_runs import _finish, _parse, _record
+from test_gpu_runs import _f, _finish, _parse, _record
 
 pytestmark = pytest.mark.gpu
+
+
+def _long_lines(target, count, width):
+    """Lines from corner to corner of a 50000x60000 viewport on a target of
+    its top 16 rows."""
+    L = pf.lib()
+    w, h = 50000, 16
+    buf = np.full((w * h + 16) * 8, 7, np.uint8)
+    ctx = C.c_void_p(L.pfCreateContext(buf.ctypes.data, w, h, *target))
+    L.pfMakeCurrent(ctx)
+    rng = np.random.default_rng(11)
+    L.pfViewport(0, 0, w, 60000)
+    L.pfMatrixMode(1)
+    L.pfLoadIdentity()
+    L.pfFrustum(*_f(-0.4, 0.4, -0.4, 0.4, 0.5, 20.0))
+    L.pfMatrixMode(0)
+    L.pfLoadIdentity()
+    L.pfDisable(0x10)
+    L.pfClear(3)
+    L.pfLineWidth(*_f(width))
+    L.pfBegin(1)
+    for k in range(count):
+        for end in (1, -1) if k % 2 else (-1, 1):
+            z = -rng.uniform(1, 3)
+            x, y = end * rng.uniform(0.9, 0.999), (end if k % 4 < 2 else -end) * (1.0 - rng.uniform(0, 1e-4))
+            L.pfColor4ub(*rng.integers(0, 256, 4).tolist())
+            L.pfVertex3f(*_f(x * 0.8 * -z, y * 0.8 * -z, z))
+    L.pfEnd()
+    assert L.pfGetError() == 0
+    return ctx, buf
+
+
+@pytest.mark.parametrize("target", [(7, 0), (7, 9)], ids=["rgba8", "rgba_half"])
+@pytest.mark.parametrize("count,width", [(8, 1.0), (8, 5.0), (2100, 1.0)])
+def test_long_lines_match_oracle(count, width, target):
+    with OracleExecutor():
+        ctx, want = _long_lines(target, count, width)
+        _finish(ctx)
+    pf.lib().pfxSetExecutor(None, None)
+    ctx, got = _long_lines(target, count, width)
+    _finish(ctx)
+    drawn = np.count_nonzero(want != np.roll(want, 8))
+    print(count, width, target, drawn, flush=True)
+    bad = np.count_nonzero(want != got)
+    assert drawn > 50 and bad == 0, f"{bad} bytes differ"
 
 
 DEPTH_FUNC, BLEND_MODE, STATE_WORDS = 49, 50, 232       # PFFstate, in words
