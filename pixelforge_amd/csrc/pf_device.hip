@@ -4116,7 +4116,6 @@ struct DLnOp {
     uint32_t  target;             // PFF_TARGET_* of color
     uint32_t  W, H, tilesX, tilesY;
     uint32_t  first, last;        // job line indices
-    uint32_t  crowded;            // as DPtOp (host)
     RunMarks  marks;
 };
 
@@ -5101,6 +5100,13 @@ bool marks_pay(uint32_t n, uint32_t tiles) {
     return n >= 2048u || (n >= 512u && (uint64_t)n * tiles >= (uint64_t)2 << 20);
 }
 constexpr size_t RUN_MARK_WORDS = (size_t)16 << 20;    // at most 64 MiB of marks
+
+// Runs whose primitives mark most tiles get none: points so large, from their
+// sizes.  Where lines end up is known on the device alone; those that mark all
+// columns of their rows (they wrap at a side of the target) still gain: 20k
+// lines from side to side at 1280x720 13.1 -> 7.9 ms a frame, 600 0.86 -> 0.76.
+bool crowded(const DPtOp& d) { return d.crowded != 0u; }
+bool crowded(const DLnOp&) { return false; }
 
 // Automatic configuration from the first pass's counts at 8x8 tiles: while
 // raster triangles span more than 32 tiles on average, tiles double in
@@ -6304,7 +6310,7 @@ int job_plan(PFDjob* J, const PFFframe* frames, uint32_t count, bool wantVid, bo
             eachRun([&](auto& d, uint32_t& most) {
                 const uint32_t n = d.last - d.first, tiles = d.tilesX * d.tilesY;
                 d.marks.words = 0;
-                if (d.crowded || !marks_pay(n, tiles)) return;
+                if (crowded(d) || !marks_pay(n, tiles)) return;
                 d.marks.shift = shift;
                 d.marks.words = ((n + 2047u) / 2048u + (1u << shift) - 1u) >> shift;
                 markWords += (size_t)tiles * d.marks.words;
