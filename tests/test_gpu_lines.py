@@ -70,6 +70,7 @@ def test_states_that_are_no_enum_values_match_oracle(func, mode):
         states = np.ctypeslib.as_array(C.cast(frame.states, C.POINTER(C.c_uint32)), (frame.numStates, STATE_WORDS))
         states[:, 48] |= 0xC                            # depth test and blending
         states[:, DEPTH_FUNC], states[:, BLEND_MODE] = func, mode
+        frame.cmds[0].clearDepth = -2.0                 # the last function is "greater or equal"
         return run.execute(C.byref(frame))
 
     L = pf.lib()
@@ -79,6 +80,6 @@ def test_states_that_are_no_enum_values_match_oracle(func, mode):
         with on_frame(run):
             _finish(ctx)
         out.append(buf)
-    assert np.count_nonzero(out[0] != 7) > 90 * 60
+    assert len(np.unique(out[0].view(np.uint32))) > 100
     bad = np.count_nonzero(out[0] != out[1])
     assert bad == 0, f"{bad} bytes differ"
