@@ -154,6 +154,70 @@ def _jobs_match_oracle(record, size, what):
         L.pfMakeCurrent(None)
 
 
+def _record_lit(seed, size, target, model, textured):
+    """Layers of lit triangles, back to front and front to back, a third of
+    the runs blended, some without lighting."""
+    L = pf.lib()
+    L.pfGenTexture.restype = C.c_void_p
+    w, h = size
+    buf = np.full((w * h + 16) * 8, 9, np.uint8)
+    ctx = C.c_void_p(L.pfCreateContext(buf.ctypes.data, w, h, *target))
+    L.pfMakeCurrent(ctx)
+    rng = np.random.default_rng(seed)
+    L.pfDisable(0x10)
+    L.pfEnable(0x8)
+    L.pfClear(3)
+    L.pfMatrixMode(1)
+    L.pfLoadIdentity()
+    L.pfFrustum(*_f(-0.4, 0.4, -0.4, 0.4, 0.5, 20.0))
+    L.pfMatrixMode(0)
+    L.pfLoadIdentity()
+    L.pfLightModel(model)
+    for k in range(3):
+        L.pfLightfv(k, 7, (C.c_float * 3)(*rng.uniform(-2, 2, 3)))
+        L.pfLightfv(k, 3, (C.c_float * 3)(*rng.uniform(0.2, 0.7, 3)))
+        L.pfLightfv(k, 4, (C.c_float * 3)(*rng.uniform(0.1, 0.5, 3)))
+        L.pfEnableLight(k)
+    L.pfMaterialfv(2, 4, (C.c_float * 3)(0.8, 0.7, 0.9))
+    L.pfMaterialf(2, 6, C.c_float(16.0))
+    if textured:
+        texels = rng.integers(0, 2**32, (17, 33), np.uint32)
+        tex = C.c_void_p(L.pfGenTexture(C.c_void_p(texels.ctypes.data), 33, 17, 7, 0))
+        L.pfTextureParameter(tex, pf.PF_REPEAT, pf.PF_BILINEAR)
+        L.pfBindTexture(tex)
+        KEEP.append(texels)
+    for _ in range(120):
+        (L.pfEnable if textured and rng.random() < 0.8 else L.pfDisable)(0x1)
+        (L.pfEnable if rng.random() < 0.8 else L.pfDisable)(0x40)
+        (L.pfEnable if rng.random() < 0.33 else L.pfDisable)(0x4)
+        L.pfBlendFunc(int(rng.integers(0, 8)))
+        L.pfDepthFunc(int(rng.choice([LESS, LESS, LESS, LEQUAL, 0])))
+        size_k, far = rng.choice([0.1, 0.5, 2.0]), rng.uniform(-0.9, 0.9)
+        L.pfBegin(2)
+        for _ in range(20):
+            c = rng.uniform(-1, 1, 2)
+            for _ in range(3):
+                z = -3.0 + 2.0 * (far + rng.uniform(-0.05, 0.05))
+                x, y = c + size_k * rng.uniform(-1, 1, 2)
+                L.pfColor4ub(*rng.integers(0, 256, 4).tolist())
+                L.pfNormal3f(*_f(*rng.normal(0, 1, 3)))
+                L.pfTexCoord2f(*_f(*rng.uniform(-2, 3, 2)))
+                L.pfVertex3f(*_f(-x * z, -y * z, z))
+        L.pfEnd()
+    assert L.pfGetError() == 0
+    return ctx, buf
+
+
+KEEP = []                                                         # texels of recorded frames
+
+
+@pytest.mark.parametrize("target", [(7, 0), (7, 9)], ids=["rgba8", "rgba_half"])
+@pytest.mark.parametrize("model,textured", [(1, False), (1, True), (0, True)], ids=["phong", "phong_tex", "gouraud_tex"])
+def test_lit_and_textured_layers_match_oracle(model, textured, target):
+    size = (101, 75)
+    _jobs_match_oracle(lambda: _record_lit(7, size, target, model, textured), size, f"model {model} {textured} {target}")
+
+
 def _weights(corners, w, h):
     """Edge values of a triangle of screen corners at pixel (0, 0), its
     largest magnitude of one within 128 pixels of the target, and their sum."""
