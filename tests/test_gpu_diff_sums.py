@@ -1,8 +1,8 @@
 """Gradients gathered per 16x16 block before they go to memory, at the sizes
 where the gathering can go wrong: more texels or vertices in a block than
 its tables hold, every pixel of a block on one triangle and few texels,
-target sides that leave part of a block empty, all light slots in use.  The
-adjoint is compared with the FP64 oracle of the same frame: relative error
+target sides that leave part of a block empty, all eight light slots in use.
+The adjoint is compared with the FP64 oracle of the same frame: relative error
 <= 1e-3 per gradient, by norm and by element, the suite's bound for FP32
 sums."""
 import numpy as np
@@ -26,11 +26,9 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("case", list(CASES))
-def test_gathered_gradients_match_fp64(case):
+def _check(s):
     if pf.lib().pfdInit() != 0:
         pytest.fail("no GPU: " + pf.lib().pfdLastError().decode())
-    s = Scene(**CASES[case])
     try:
         job = oracle_job(s)
         s.rerecord()
@@ -48,3 +46,19 @@ def test_gathered_gradients_match_fp64(case):
             assert np.abs(a - b).max() <= REL * np.abs(b).max(), name
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_gathered_gradients_match_fp64(case):
+    _check(Scene(**CASES[case]))
+
+
+@pytest.mark.parametrize("textured", [True, False])
+def test_all_light_slots_match_fp64(textured):
+    s = Scene(width=50, height=30, nx=6, nz=6, lights=4, attenuation=True, textured=textured, seed=28)
+    rng = np.random.default_rng(28)
+    s.light_ids = list(range(8))
+    s.light_pos = (rng.uniform(-1, 1, (8, 3)) + [0, 0, -1.0]).astype(np.float32)
+    s.ldiff = rng.uniform(0.03, 0.12, (8, 3)).astype(np.float32)
+    s.lspec = rng.uniform(0.02, 0.08, (8, 3)).astype(np.float32)
+    _check(s)
