@@ -4984,9 +4984,9 @@ bool upload_ready(PFDjob* J) {
     return true;
 }
 
-// Host -> device, in order with the job's stream.  Small sources are read
-// before it returns; page-locked ones above UP_SMALL are read by the next
-// upload_flush's kernel, and must stay as they are until the stream has been
+// Host -> device, in order with the job's stream.  Ordinary memory is read
+// before it returns; page-locked memory, read by the next upload_flush's kernel
+// or by a copy command, must stay as it is until the stream has been
 // synchronised.  Kernels that read `dev` are launched after upload_flush.
 int upload(PFDjob* J, void* dev, const void* host, size_t bytes) {
     if (bytes == 0) return PFD_OK;
@@ -5013,7 +5013,8 @@ int upload(PFDjob* J, void* dev, const void* host, size_t bytes) {
         return PFD_OK;
     }
     if ((rc = upload_flush(J))) return rc;
-    HIP_TRY(staged_h2d(J, dev, host, bytes), PFD_E_LAUNCH);
+    if (host_pinned(host)) HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, J->stream), PFD_E_LAUNCH);
+    else HIP_TRY(staged_h2d(J, dev, host, bytes), PFD_E_LAUNCH);
     return PFD_OK;
 }
 
