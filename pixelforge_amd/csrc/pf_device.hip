@@ -2004,9 +2004,8 @@ struct RasterArgs {
 //
 // Each wave owns one 8x8 block of a tile (one pixel per lane; colour and
 // depth stay in VGPRs from the fused clear / load to the single write-back)
-// and walks the tile's pair list 64 entries at a time (32 where a lane stages
-// whole lit records at once): the lanes fetch the entries and their
-// raster-triangle records in one round trip, keep the ones whose bbox meets
+// and walks the tile's pair list 32 or 64 entries at a time: the lanes fetch
+// the entries and their raster-triangle records, keep the ones whose bbox meets
 // the block (and, in the HIZ instances, that are not behind all its pixels)
 // and stage them, compacted and still in list order, up to 32 at once, in the
 // wave's LDS.  Each staged triangle is then tested
@@ -2318,15 +2317,12 @@ __device__ __forceinline__ bool hidden_behind(uint4 q0, uint4 q1, uint4 q2, uint
 // targets, which keep in them whether a pixel was written).
 // HIZ: from the second batch of a list on, records hidden behind the pixels
 // are found before they are staged (K = 1).
-template <int MODE, bool PHONG, int K, int TK, bool QUAD, bool WIN, bool HIZ>
+// ONCE: a batch is what 32 entries leave, not filled up from the next ones.
+template <int MODE, bool PHONG, int K, int TK, bool QUAD, bool WIN, bool HIZ, bool ONCE>
 __device__ __forceinline__ uint32_t raster_block(const RasterArgs& A, const DFrame& F, const DTileFrame& sg,
                                                  uint32_t frame, int bx0, int by0, uint32_t e0, uint32_t e1,
                                                  WaveQueueT<PHONG>& Q, int qbit) {
     constexpr int PM = MODE;                      // 0 packed, 1 in place
-    // Entries read per step.  Where nothing is hidden a per-fragment lit
-    // in-place raster is 8 % faster with half of them (1080p spheres, four
-    // lights: 632 -> 585 us); everything else is up to 8 % faster with 64.
-    constexpr uint32_t STEP = PHONG && !HIZ ? 32u : 64u;
     constexpr int TW = (K == 1) ? 8 : 16;
     constexpr int RS = 64 / TW;                    // rows between a lane's pixels
     const int lane = threadIdx.x & 63;
@@ -2367,160 +2363,220 @@ __device__ __forceinline__ uint32_t raster_block(const RasterArgs& A, const DFra
     // Last column and row of the block inside the target.
     const int xLim = min(bx0 + TW - 1, (int)F.W - 1), yLim = min(by0 + TW - 1, (int)F.H - 1);
     uint32_t frags = 0;
+    // Whether a record (its leading chunks and meta) meets this block; rm: the
+    // pixels it may cover (K = 1).
+    const auto meets = [&](const uint4& q0, const uint4& q1, const uint4& q2, const uint4& q3, uint32_t meta, uint64_t& rm) {
+        const int32_t xMin = (int32_t)q2.y, yMin = (int32_t)q2.z;
+        const int32_t xMax = (int32_t)q2.w, yMax = (int32_t)q3.x;
+        bool ov = !(xMax <= bx0 || xMin > bx0 + TW - 1 || yMax < by0 || yMin > by0 + TW - 1);
+        // An edge negative over the whole block leaves it uncovered.  With
+        // NOWRAP the block (inside a tile that meets the bbox, so within 64
+        // px of it) sees no int32 wrap: its largest w is at a corner.
+        if (ov && (meta & META_NOWRAP)) {
+            const int32_t xs[2] = { bx0, bx0 + TW - 1 }, ys[2] = { by0, by0 + TW - 1 };
+            const int32_t eA[3] = { (int32_t)q0.x, (int32_t)q0.y, (int32_t)q0.z };
+            const int32_t eB[3] = { (int32_t)q0.w, (int32_t)q1.x, (int32_t)q1.y };
+            const int32_t eC[3] = { (int32_t)q1.z, (int32_t)q1.w, (int32_t)q2.x };
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const int32_t hi = eA[k] * xs[eA[k] > 0] + eB[k] * ys[eB[k] > 0] + eC[k];
+                ov = ov && hi >= 0;
+            }
+        }
+        if (ov && K == 1) {
+            // The coverage rule's bbox part (x in [xMin, xMax), y in
+            // [yMin, yMax]) and the target, as a pixel mask: for exact
+            // triangles the edges imply it, for the others it is their
+            // bbox test.  An empty mask drops the record.
+            const int32_t rx0 = max(bx0, xMin), rx1 = min(xLim, xMax - 1);
+            const int32_t ry0 = max(by0, yMin), ry1 = min(yLim, yMax);
+            if (rx0 > rx1 || ry0 > ry1) ov = false;
+            else rm = rect_mask8(rx0 - bx0, rx1 - bx0, ry0 - by0, ry1 - by0);
+        }
+        return ov;
+    };
+    const auto stage_light = [&](int slot, uint32_t r, uint32_t meta) {
+        if constexpr (PHONG) {
+            if (meta & META_PHONG) {
+                const uint4* ls = reinterpret_cast<const uint4*>(&A.rtl[r]);
+                uint4* ld = reinterpret_cast<uint4*>(&Q.recL[slot][0]);
+#pragma unroll
+                for (int k = 0; k < 5; k++) ld[k] = ls[k];
+            }
+        }
+    };
     for (uint32_t e = e0; e < e1;) {
-        // Stages up to 32 records that meet this block, in list order: STEP
-        // list entries are read at a time (with QUAD, those holding the
-        // block's quadrant bit, compacted through the queue's colour and
-        // depth slots, which are free here), a lane fetching and testing one
-        // record each, until the batch is full or the list ends.
         uint32_t nt = 0;
         // 24-bit edge multiplies for the whole batch when every staged
         // record allows them (decided before the loop: no per-record branch).
-        bool allSmall = true;
-        // Hidden records: those no sample of which can pass its depth test
-        // against the block's pixels as they are now.  A LESS or LEQUAL record
-        // stays hidden unless a record before it in the batch may raise a
-        // pixel's depth (mayRaise), a GREATER or GEQUAL one unless one may
-        // lower it.
-        // Only from the second batch on: the first one meets the cleared
-        // pixels.
-        const bool hide = HIZ && e != e0;
-        bool mayRaise = false, mayLower = false, anyHidden = false;
-        while (nt < (uint32_t)BATCH && e < e1) {
-            uint32_t nb = 0, r = 0;                // entries read; the lane's raster triangle
-            const uint32_t first = e;
-            uint32_t* const ids = Q.fcol;          // QUAD: raster triangles, and the list positions after them
-            uint32_t* const pos = reinterpret_cast<uint32_t*>(Q.fz);
+        bool allSmall = true, anyHidden = false;
+        if constexpr (ONCE) {
+            // The batch is what meets the block of the next 32 entries (with QUAD
+            // of the next 32 holding the block's quadrant bit, read 64 at a time
+            // and compacted in list order through the queue's record-id slots),
+            // a lane fetching a whole record.
+            uint32_t nb = 0, r = 0;
             if constexpr (QUAD) {
-                while (nb < STEP && e < e1) {
+                while (nb < (uint32_t)BATCH && e < e1) {
                     const bool has = e + (uint32_t)lane < e1;
                     const uint32_t v = has ? A.vals[e + lane] : 0u;
                     const bool mine = has && ((v >> (PAIR_QUAD_SH + (uint32_t)qbit)) & 1u);
                     const uint64_t M = __builtin_amdgcn_ballot_w64(mine);
-                    const uint32_t room = STEP - nb, found = (uint32_t)__popcll(M);
+                    const uint32_t room = (uint32_t)BATCH - nb, found = (uint32_t)__popcll(M);
                     const uint32_t rank = (uint32_t)lane_rank(M);
-                    if (mine && rank < room) { ids[nb + rank] = v & PAIR_RT_MASK; pos[nb + rank] = e + (uint32_t)lane + 1u; }
+                    if (mine && rank < room) Q.recId[nb + rank] = v & PAIR_RT_MASK;
                     if (found > room) {
-                        // Full: continue after its last entry.
+                        // The batch fills here: continue after its last entry.
                         e += (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(mine && rank == room - 1u)) + 1u;
-                        nb = STEP;
+                        nb = (uint32_t)BATCH;
                     } else {
                         e += min(64u, e1 - e);
                         nb += found;
                     }
                 }
                 wave_sync();
-                if ((uint32_t)lane < nb) r = ids[lane];
+                if ((uint32_t)lane < nb) r = Q.recId[lane];
+                wave_sync();
             } else {
-                nb = min(STEP, e1 - e);
-                if ((uint32_t)lane < nb) r = A.vals[e + lane] & PAIR_RT_MASK;
-                e += nb;
+                nb = min((uint32_t)BATCH, e1 - e);
             }
-            // Their records; keep the ones that meet this block, compacted in
-            // list order.
             bool ov = false;
-            // (What the tests read of a record is loaded first; the rest of the
-            // kept ones when they are staged, so that it takes no registers
-            // meanwhile.  With 32 per step all of it at once.)
             const uint4 z4 = make_uint4(0u, 0u, 0u, 0u);
             uint4 q0 = z4, q1 = z4, q2 = z4, q3 = z4, q4 = z4, q5 = z4, q6 = z4, q7 = z4;
-            uint32_t z2 = 0u, meta = 0u;
             uint64_t rm = 0;
-            const uint4* src = reinterpret_cast<const uint4*>(&A.rts[r]);
             if ((uint32_t)lane < nb) {
+                if constexpr (!QUAD) r = A.vals[e + lane] & PAIR_RT_MASK;
+                const uint4* src = reinterpret_cast<const uint4*>(&A.rts[r]);
                 q0 = src[0]; q1 = src[1]; q2 = src[2]; q3 = src[3];
-                if (STEP == 32u) { q4 = src[4]; q5 = src[5]; q6 = src[6]; q7 = src[7]; z2 = q4.x; meta = q5.x; }
-                else { z2 = src[4].x; meta = src[5].x; }
-                const int32_t xMin = (int32_t)q2.y, yMin = (int32_t)q2.z;
-                const int32_t xMax = (int32_t)q2.w, yMax = (int32_t)q3.x;
-                ov = !(xMax <= bx0 || xMin > bx0 + TW - 1 || yMax < by0 || yMin > by0 + TW - 1);
-                // An edge negative over the whole block leaves it uncovered.  With
-                // NOWRAP the block (inside a tile that meets the bbox, so within 64
-                // px of it) sees no int32 wrap: its largest w is at a corner.
-                if (ov && (meta & META_NOWRAP)) {
-                    const int32_t xs[2] = { bx0, bx0 + TW - 1 }, ys[2] = { by0, by0 + TW - 1 };
-                    const int32_t eA[3] = { (int32_t)q0.x, (int32_t)q0.y, (int32_t)q0.z };
-                    const int32_t eB[3] = { (int32_t)q0.w, (int32_t)q1.x, (int32_t)q1.y };
-                    const int32_t eC[3] = { (int32_t)q1.z, (int32_t)q1.w, (int32_t)q2.x };
-#pragma unroll
-                    for (int k = 0; k < 3; k++) {
-                        const int32_t hi = eA[k] * xs[eA[k] > 0] + eB[k] * ys[eB[k] > 0] + eC[k];
-                        ov = ov && hi >= 0;
-                    }
-                }
-                if (ov && K == 1) {
-                    // The coverage rule's bbox part (x in [xMin, xMax), y in
-                    // [yMin, yMax]) and the target, as a pixel mask: for exact
-                    // triangles the edges imply it, for the others it is their
-                    // bbox test.  An empty mask drops the record.
-                    const int32_t rx0 = max(bx0, xMin), rx1 = min(xLim, xMax - 1);
-                    const int32_t ry0 = max(by0, yMin), ry1 = min(yLim, yMax);
-                    if (rx0 > rx1 || ry0 > ry1) ov = false;
-                    else rm = rect_mask8(rx0 - bx0, rx1 - bx0, ry0 - by0, ry1 - by0);
-                }
-            }
-            // Records hidden behind the block's pixels: one that covers the
-            // whole block is dropped (its samples are counted below), a
-            // partly covering one is staged for its count alone.
-            uint32_t idFlag = 0u;
-            bool dropped = false;
-            if (__builtin_expect(hide, 0)) {
-                const uint32_t f = (meta >> META_DFUNC_SH) & 7u;
-                const bool test = (meta & META_DEPTH) != 0u;
-                mayRaise = mayRaise || __builtin_amdgcn_ballot_w64(ov && (!test || f >= 4u)) != 0ull;
-                mayLower = mayLower || __builtin_amdgcn_ballot_w64(ov && (!test || f == 2u || f == 3u)) != 0ull;
-                if (!(mayRaise && mayLower)) {                  // uniform over the wavefront
-                    // Depths of GREATER and GEQUAL tests are negated.
-                    const float sign = mayRaise ? -1.0f : 1.0f;
-                    const float dep0 = wave_max(in[0] ? sign * dep[0] : -__builtin_inff());
-                    bool full = false, hid = false;
-                    if (ov && test && f >= 2u && (meta & META_NOWRAP))
-                        hid = hidden_behind(q0, q1, q2, q3, z2, bx0, by0, sign, dep0, full);
-                    dropped = hid && full;
-                    if (hid) idFlag = REC_HIDDEN;
-                    ov = ov && !dropped;
-                }
+                q4 = src[4]; q5 = src[5]; q6 = src[6]; q7 = src[7];
+                ov = meets(q0, q1, q2, q3, q5.x, rm);
             }
             const uint64_t OV = __builtin_amdgcn_ballot_w64(ov);
-            const uint32_t room = (uint32_t)BATCH - nt, found = (uint32_t)__popcll(OV);
-            const uint32_t rank = (uint32_t)lane_rank(OV);
-            const bool put = ov && rank < room;
-            allSmall = allSmall && __builtin_amdgcn_ballot_w64(put && !(meta & META_SMALL)) == 0ull;
-            if (put) {
-                const int slot = (int)(nt + rank);
+            nt = (uint32_t)__popcll(OV);
+            allSmall = __builtin_amdgcn_ballot_w64(ov && !(q5.x & META_SMALL)) == 0ull;
+            if (ov) {
+                const int slot = lane_rank(OV);
                 uint4* dst = reinterpret_cast<uint4*>(&Q.rec[slot][0]);
                 dst[0] = q0; dst[1] = q1; dst[2] = q2; dst[3] = q3;
-                if (STEP == 32u) {
-                    dst[4] = q4; dst[5] = q5; dst[6] = q6; dst[7] = q7;
-                } else {
-                    asm volatile("" ::: "memory"); // the chunks above leave their registers first
-                    dst[4] = src[4]; dst[5] = src[5]; dst[6] = src[6]; dst[7] = src[7];
-                }
-                Q.recId[slot] = r | idFlag;
+                dst[4] = q4; dst[5] = q5; dst[6] = q6; dst[7] = q7;
+                Q.recId[slot] = r;
                 if (K == 1) Q.rmask[slot] = rm;
-                if constexpr (PHONG) {
-                    if (meta & META_PHONG) {
-                        const uint4* ls = reinterpret_cast<const uint4*>(&A.rtl[r]);
-                        uint4* ld = reinterpret_cast<uint4*>(&Q.recL[slot][0]);
-#pragma unroll
-                        for (int k = 0; k < 5; k++) ld[k] = ls[k];
+                stage_light(slot, r, q5.x);
+            }
+            if constexpr (!QUAD) e += (uint32_t)BATCH;
+        } else {
+            // Stages up to 32 records that meet the block, in list order: 64 list
+            // entries are read at a time (with QUAD, those holding the block's
+            // quadrant bit, compacted through the queue's colour and depth slots,
+            // which are free here), a lane fetching and testing one record each,
+            // until the batch is full or the list ends.
+            constexpr uint32_t STEP = 64u;
+            // Hidden records: those no sample of which can pass its depth test
+            // against the block's pixels as they are now.  A LESS or LEQUAL record
+            // stays hidden unless a record before it in the batch may raise a
+            // pixel's depth (mayRaise), a GREATER or GEQUAL one unless one may
+            // lower it.
+            // Only from the second batch on: the first one meets the cleared
+            // pixels.
+            const bool hide = HIZ && e != e0;
+            bool mayRaise = false, mayLower = false;
+            while (nt < (uint32_t)BATCH && e < e1) {
+                uint32_t nb = 0, r = 0;                // entries read; the lane's raster triangle
+                const uint32_t first = e;
+                uint32_t* const ids = Q.fcol;          // QUAD: raster triangles, and the list positions after them
+                uint32_t* const pos = reinterpret_cast<uint32_t*>(Q.fz);
+                if constexpr (QUAD) {
+                    while (nb < STEP && e < e1) {
+                        const bool has = e + (uint32_t)lane < e1;
+                        const uint32_t v = has ? A.vals[e + lane] : 0u;
+                        const bool mine = has && ((v >> (PAIR_QUAD_SH + (uint32_t)qbit)) & 1u);
+                        const uint64_t M = __builtin_amdgcn_ballot_w64(mine);
+                        const uint32_t room = STEP - nb, found = (uint32_t)__popcll(M);
+                        const uint32_t rank = (uint32_t)lane_rank(M);
+                        if (mine && rank < room) { ids[nb + rank] = v & PAIR_RT_MASK; pos[nb + rank] = e + (uint32_t)lane + 1u; }
+                        if (found > room) {
+                            // Full: continue after its last entry.
+                            e += (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(mine && rank == room - 1u)) + 1u;
+                            nb = STEP;
+                        } else {
+                            e += min(64u, e1 - e);
+                            nb += found;
+                        }
+                    }
+                    wave_sync();
+                    if ((uint32_t)lane < nb) r = ids[lane];
+                } else {
+                    nb = min(STEP, e1 - e);
+                    if ((uint32_t)lane < nb) r = A.vals[e + lane] & PAIR_RT_MASK;
+                    e += nb;
+                }
+                // Their records; keep the ones that meet this block, compacted in
+                // list order.  What the tests read of a record is loaded first; the
+                // rest of the kept ones when they are staged, so that it takes no
+                // registers meanwhile.
+                bool ov = false;
+                const uint4 z4 = make_uint4(0u, 0u, 0u, 0u);
+                uint4 q0 = z4, q1 = z4, q2 = z4, q3 = z4;
+                uint32_t z2 = 0u, meta = 0u;
+                uint64_t rm = 0;
+                const uint4* src = reinterpret_cast<const uint4*>(&A.rts[r]);
+                if ((uint32_t)lane < nb) {
+                    q0 = src[0]; q1 = src[1]; q2 = src[2]; q3 = src[3];
+                    z2 = src[4].x; meta = src[5].x;
+                    ov = meets(q0, q1, q2, q3, meta, rm);
+                }
+                // Records hidden behind the block's pixels: one that covers the
+                // whole block is dropped (its samples are counted below), a
+                // partly covering one is staged for its count alone.
+                uint32_t idFlag = 0u;
+                bool dropped = false;
+                if (__builtin_expect(hide, 0)) {
+                    const uint32_t f = (meta >> META_DFUNC_SH) & 7u;
+                    const bool test = (meta & META_DEPTH) != 0u;
+                    mayRaise = mayRaise || __builtin_amdgcn_ballot_w64(ov && (!test || f >= 4u)) != 0ull;
+                    mayLower = mayLower || __builtin_amdgcn_ballot_w64(ov && (!test || f == 2u || f == 3u)) != 0ull;
+                    if (!(mayRaise && mayLower)) {                  // uniform over the wavefront
+                        // Depths of GREATER and GEQUAL tests are negated.
+                        const float sign = mayRaise ? -1.0f : 1.0f;
+                        const float dep0 = wave_max(in[0] ? sign * dep[0] : -__builtin_inff());
+                        bool full = false, hid = false;
+                        if (ov && test && f >= 2u && (meta & META_NOWRAP))
+                            hid = hidden_behind(q0, q1, q2, q3, z2, bx0, by0, sign, dep0, full);
+                        dropped = hid && full;
+                        if (hid) idFlag = REC_HIDDEN;
+                        ov = ov && !dropped;
                     }
                 }
+                const uint64_t OV = __builtin_amdgcn_ballot_w64(ov);
+                const uint32_t room = (uint32_t)BATCH - nt, found = (uint32_t)__popcll(OV);
+                const uint32_t rank = (uint32_t)lane_rank(OV);
+                const bool put = ov && rank < room;
+                allSmall = allSmall && __builtin_amdgcn_ballot_w64(put && !(meta & META_SMALL)) == 0ull;
+                if (put) {
+                    const int slot = (int)(nt + rank);
+                    uint4* dst = reinterpret_cast<uint4*>(&Q.rec[slot][0]);
+                    dst[0] = q0; dst[1] = q1; dst[2] = q2; dst[3] = q3;
+                    asm volatile("" ::: "memory");     // the chunks above leave their registers first
+                    dst[4] = src[4]; dst[5] = src[5]; dst[6] = src[6]; dst[7] = src[7];
+                    Q.recId[slot] = r | idFlag;
+                    if (K == 1) Q.rmask[slot] = rm;
+                    stage_light(slot, r, meta);
+                }
+                if (HIZ) anyHidden = anyHidden || __builtin_amdgcn_ballot_w64(put && idFlag) != 0ull;
+                int last = 63;                         // the last lane whose record this batch has dealt with
+                if (found > room) {
+                    // The batch is full: the list continues after its last record.
+                    last = __builtin_ctzll(__builtin_amdgcn_ballot_w64(ov && rank == room - 1u));
+                    e = QUAD ? (uint32_t)__builtin_amdgcn_readfirstlane(pos[last]) : first + (uint32_t)last + 1u;
+                    nt = (uint32_t)BATCH;
+                } else {
+                    nt += found;
+                }
+                if (HIZ && __builtin_amdgcn_ballot_w64(dropped))
+                    frags += (uint32_t)__builtin_amdgcn_readlane(
+                        wave_incl_scan(dropped && lane <= last ? (uint32_t)__popcll(rm) : 0u), 63);
+                if constexpr (QUAD) wave_sync();       // ids and pos are written again
             }
-            if (HIZ) anyHidden = anyHidden || __builtin_amdgcn_ballot_w64(put && idFlag) != 0ull;
-            int last = 63;                         // the last lane whose record this batch has dealt with
-            if (found > room) {
-                // The batch is full: the list continues after its last record.
-                last = __builtin_ctzll(__builtin_amdgcn_ballot_w64(ov && rank == room - 1u));
-                e = QUAD ? (uint32_t)__builtin_amdgcn_readfirstlane(pos[last]) : first + (uint32_t)last + 1u;
-                nt = (uint32_t)BATCH;
-            } else {
-                nt += found;
-            }
-            if (HIZ && __builtin_amdgcn_ballot_w64(dropped))
-                frags += (uint32_t)__builtin_amdgcn_readlane(
-                    wave_incl_scan(dropped && lane <= last ? (uint32_t)__popcll(rm) : 0u), 63);
-            if constexpr (QUAD) wave_sync();       // ids and pos are written again
         }
         wave_sync();
         int nf = 0;
@@ -2674,7 +2730,14 @@ __device__ __forceinline__ void raster_tiles(const RasterArgs& A) {
         // (1080p frame: raster 100 -> 95 us; 4K frame 548 -> 484 us); in
         // place, whose large triangles meet every quadrant, it only costs.
         constexpr bool QUAD = TS == 16 && K == 1 && MODE == 0;
-        frags += raster_block<MODE, PHONG, K, TK, QUAD, WIN, HIZ>(A, F, sg, frame, bx0, by0, e0, e1, Q, b);
+        // How a batch is staged, without HIZ (whole replays, one way against
+        // the other): filling it up wins where a block skips most of its
+        // tile's list (32x32 tiles, packed: 338 -> 280 and 222 -> 191 us) and
+        // for unlit triangles in place (2-3 %); taking 32 entries as they are
+        // where the list is the block's own (packed, 8x8 and 16x16 tiles: 2-5 %
+        // on spheres and height fields) and for lit fragments in place (1-6 %).
+        constexpr bool ONCE = !HIZ && (MODE == 0 ? TS <= 16 && (K == 1 || PHONG) : PHONG);
+        frags += raster_block<MODE, PHONG, K, TK, QUAD, WIN, HIZ, ONCE>(A, F, sg, frame, bx0, by0, e0, e1, Q, b);
     }
     count(frags);
 }
@@ -5079,15 +5142,19 @@ void launch_raster_ts(const RasterArgs& ra, uint32_t shift, uint32_t numTiles, b
 // Whether a pass's raster looks for hidden records (HIZ): where tiles hold
 // many triangles on average -- fewer of them where they span several tiles
 // each, so that they lie in layers and not side by side -- or where each
-// fragment is lit.  Its code costs 4-8 % where tiles hold few (1080p height
-// field, 48 pairs per 16x16 tile, 2.6 per triangle: 121 -> 130 us) and gains
-// as the layers grow: random triangles at 1280x720, 16x16 tiles, packed, 26
-// large ones per tile 57.5 -> 57.4 us, 54 104 -> 94, 117 197 -> 122; 68
-// small ones 63 -> 61, 272 200 -> 174; 800x600, 2688 large ones, in place
-// 1755 -> 525 us.  1080p spheres, four lights per fragment, packed, 34 pairs
-// per tile 173 -> 170 us (4K frame 526 -> 480), but in place 590 -> 620.
-bool hidden_pays(uint64_t pairs, uint32_t numRT, uint32_t tiles, bool phong, uint32_t mode) {
-    return (phong && mode == 0u) || pairs >= (uint64_t)(pairs > (uint64_t)4 * numRT ? 48 : 128) * tiles;
+// fragment is lit and packed and an 8x8 block has about eight records to look
+// at (24 pairs a tile above 8x8).  Its code costs 4-8 % where tiles hold few
+// (1080p height field, 48 pairs per 16x16 tile, 2.6 per triangle: 121 -> 130
+// us) and gains as the layers grow: random triangles at 1280x720, 16x16 tiles,
+// packed, 26 large ones per tile 57.5 -> 57.4 us, 54 104 -> 94, 117 197 -> 122;
+// 68 small ones 63 -> 61, 272 200 -> 174; 800x600, 2688 large ones, in place
+// 1755 -> 540 us.  Spheres lit per fragment, packed, 16x16 tiles, whole replay
+// against the one without: 640x480, 8 pairs per tile +2 %; 1080p, 31-34 pairs,
+// eight scenes of 1-4 lights -12 to +6 %, -5 % on average; 4K, 51 pairs -15 to
+// -17 %.  In place 590 -> 620 us.
+bool hidden_pays(uint64_t pairs, uint32_t numRT, uint32_t tiles, uint32_t shift, bool phong, uint32_t mode) {
+    if (phong && mode == 0u && pairs >= (uint64_t)(shift == 3 ? 8 : 24) * tiles) return true;
+    return pairs >= (uint64_t)(pairs > (uint64_t)4 * numRT ? 48 : 128) * tiles;
 }
 
 void layout_tiles(PFDjob* J);
@@ -5209,7 +5276,7 @@ void launch_pass_raster(PFDjob* J, const PassInfo& P, const uint32_t* vals, size
     ra.winner = J->diff ? (uint32_t*)J->winner.p : nullptr;
     ra.clearSnap = (const uint32_t*)J->clearSnap.p;
     const int tk = target_class(J);
-    const bool hiz = hidden_pays(P.numPairs, P.numRT, J->numTiles, J->anyPhong, J->cfg.rasterMode & 1u);
+    const bool hiz = hidden_pays(P.numPairs, P.numRT, J->numTiles, J->tileShift, J->anyPhong, J->cfg.rasterMode & 1u);
     switch (J->cfg.rasterMode) {
     case 1: launch_raster_ts<1, 1>(ra, J->tileShift, J->numTiles, J->anyPhong, tk, hiz, J->stream); break;
     case 2: launch_raster_ts<0, 4>(ra, J->tileShift, J->numTiles, J->anyPhong, tk, hiz, J->stream); break;
