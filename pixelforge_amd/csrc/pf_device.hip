@@ -7037,10 +7037,16 @@ int diff_args(PFDjob* J, const PFDdiffParams* p, DiffArgs& a) {
 
 dim3 diff_grid(const DiffArgs& a) { return dim3((a.W + 15) / 16, (a.H + 15) / 16); }
 
-// The integer pass that fixes coverage and winners; runs once per job.
+// The integer pass that fixes coverage and winners; runs once per job.  Tiles
+// without triangles in a frame without a clear are not drawn: the winners of
+// their pixels are cleared here.
 int diff_raster(PFDjob* J) {
     if (J->diffRan) return PFD_OK;
     int rc;
+    const uint32_t npx = J->frames[0].W * J->frames[0].H;
+    hipLaunchKernelGGL(k_fill_u32, dim3(std::min(4096u, grid_for(npx, 256 * 4))), dim3(256), 0, J->stream,
+                       (uint32_t*)J->winner.p, npx, 0u);
+    HIP_TRY(hipGetLastError(), PFD_E_LAUNCH);
     if ((rc = pfdJobUploadTargets(J)) || (rc = run_all(J, true))) return rc;
     if ((rc = pfdJobDownload(J))) return rc;
     J->diffRan = true;
