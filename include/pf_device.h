@@ -106,7 +106,9 @@ int pfdExecuteFrames(const PFFframe* frames, uint32_t count);
  * its raster pass (a 1920x1080 frame of 200k textured triangles needs about
  * 75 MB).  Calls on one GPU share that array, which keeps the last call's
  * contents; overlapping calls would race on it, so the library serialises
- * the calls of a process with a lock.  Results equal pfdExecuteFrame's. */
+ * the calls of a process with a lock.  Results equal pfdExecuteFrame's; the
+ * page-locked upload block, the download kernel and the marks of long point
+ * and line runs, which that allocates for speed, are left out. */
 #define PFD_SCRATCH_BYTES_MIB 128
 int pfdExecuteFrameNoAlloc(const PFFframe* frame);
 

@@ -3712,7 +3712,7 @@ __device__ __forceinline__ uint32_t compact_hits(bool hit, const REC& r, REC* ou
 // the projection); the tile then tests only the groups marked for it,
 // instead of the whole run.  1080p, 100k points (391 steps of 256 per tile,
 // about 20 groups of 64 marked): k_points 5087 -> 114 us plus 6 of marking;
-// 720p wireframe, 14k lines: k_lines 308 -> 89 us plus 32.  A run without
+// 720p wireframe, 14k lines: k_lines 308 -> 85 us plus 33.  A run without
 // marks (words = 0) has every group tested.
 struct RunMarks {
     uint32_t* bits;               // [tiles][words]

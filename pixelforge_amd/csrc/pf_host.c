@@ -343,8 +343,8 @@ static void store_release(ListStore* st);
  * array takes more than PIN_MAX, and all contexts together no more than
  * PIN_TOTAL: what does not fit stays on the heap.  Memory of which PIN_IDLE
  * frames in a row use less than a quarter is given back.
- * First frame of a process, 100k points / 50k lines at 640x480: 14.1 / 16 ms;
- * doubled from 256 elements on in page-locked memory 16.9 / 19, on the heap
+ * First frame of a process, 100k points / 50k lines at 640x480: 15.3 / 17 ms;
+ * doubled from 256 elements on in page-locked memory 16.7 / 19, on the heap
  * alone 14.5 / 31. */
 #define PIN_MIN   ((size_t)128 << 10)
 #define PIN_MAX   ((size_t)64 << 20)
